@@ -32,12 +32,7 @@ namespace {
 
 constexpr int GT = 16;            // Gram output tile (GT x GT per workgroup)
 constexpr int GROWS = 64;         // rows staged in LDS per step
-// Rows per split-K chunk of the Gram products: a multiple of 32 that gives at
-// most GCHUNKS chunks.  A chunk is one workgroup, so a fixed 4096 rows left
-// three workgroups at n = 9,125 (224 us per product, 63% of a whole solve);
-// 32 rows give 286 and 5 us.  Above 512 chunks the partial results cost more
-// to write and re-read than the extra workgroups hide (n = 2e6: 3,936 rows).
-constexpr int64_t GCHUNKS = 512;
+constexpr int64_t GCHUNK = 4096;  // rows per split-K chunk
 constexpr int EMAX = 96;          // largest subspace whose eigenproblem runs on the GPU
 constexpr int ET = 1024;          // threads of the eigensolver workgroup
 
@@ -64,14 +59,13 @@ __global__ void k_precond(int64_t n, int R, const double *hd, const double *thet
 
 // part[chunk][i + mv*j] = sum over the chunk's rows of V[r,i] W[r,j]
 __global__ __launch_bounds__(256) void k_gram_partial(int64_t n, const double *V, int mv,
-                                                      const double *W, int mw, int64_t crow,
-                                                      double *part) {
+                                                      const double *W, int mw, double *part) {
   __shared__ double sV[GROWS][GT + 1];
   __shared__ double sW[GROWS][GT + 1];
   const int tid = threadIdx.x, ti = tid % GT, tj = tid / GT;
   const int i0 = blockIdx.y * GT, j0 = blockIdx.z * GT;
-  const int64_t r_begin = (int64_t)blockIdx.x * crow;
-  const int64_t r_end = std::min<int64_t>(n, r_begin + crow);
+  const int64_t r_begin = (int64_t)blockIdx.x * GCHUNK;
+  const int64_t r_end = std::min<int64_t>(n, r_begin + GCHUNK);
   double acc = 0.0;
   for (int64_t r0 = r_begin; r0 < r_end; r0 += GROWS) {
     for (int e = tid; e < GROWS * GT; e += 256) {
@@ -90,63 +84,35 @@ __global__ __launch_bounds__(256) void k_gram_partial(int64_t n, const double *V
 }
 
 // part[chunk][i + mv*j] as k_gram_partial, for mv, mw <= GW: one workgroup
-// per row chunk covers every output, so V and W are read once.  Fewer outputs
-// than threads (the usual m x R products) are summed by several threads each,
-// over interleaved rows of the stage, and combined in thread order; without
-// that, 24 x 2 outputs left 208 of 256 threads idle behind a serial chain of
-// LDS reads.
+// per row chunk covers every output, so V and W are read once
 constexpr int GW = 64, GR = 32;
 __global__ __launch_bounds__(256) void k_gram_partial_wide(int64_t n, const double *V, int mv,
-                                                           const double *W, int mw, int64_t crow,
+                                                           const double *W, int mw,
                                                            double *part) {
-  __shared__ double sV[GW][GR + 1];
-  __shared__ double sW[GW][GR + 1];
-  __shared__ double sP[256];
+  __shared__ double sV[GR][GW + 1];
+  __shared__ double sW[GR][GW + 1];
   const int tid = threadIdx.x;
   const int cnt = mv * mw;
-  const int64_t r_begin = (int64_t)blockIdx.x * crow;
-  const int64_t r_end = std::min<int64_t>(n, r_begin + crow);
-  auto stage = [&](int64_t r0) {
-    for (int e = tid; e < GR * (mv + mw); e += 256) {
-      const int rr = e % GR, cc = e / GR;
-      const int64_t r = r0 + rr;
-      if (cc < mv) sV[cc][rr] = r < r_end ? V[r + n * cc] : 0.0;
-      else sW[cc - mv][rr] = r < r_end ? W[r + n * (cc - mv)] : 0.0;
-    }
-    __syncthreads();
-  };
-  if (2 * cnt <= 256) {
-    const int ng = 256 / cnt < GR ? 256 / cnt : GR;  // threads per output
-    const int o = tid % cnt, g = tid / cnt;
-    const int i = o % mv, j = o / mv;
-    double acc = 0.0;
-    for (int64_t r0 = r_begin; r0 < r_end; r0 += GR) {
-      stage(r0);
-      if (g < ng)
-        for (int rr = g; rr < GR; rr += ng) acc += sV[i][rr] * sW[j][rr];
-      __syncthreads();
-    }
-    sP[tid] = acc;
-    __syncthreads();
-    if (tid < cnt) {
-      double s = acc;
-      for (int k = 1; k < ng; k++) s += sP[tid + k * cnt];
-      part[(int64_t)blockIdx.x * cnt + tid] = s;
-    }
-    return;
-  }
+  const int64_t r_begin = (int64_t)blockIdx.x * GCHUNK;
+  const int64_t r_end = std::min<int64_t>(n, r_begin + GCHUNK);
   double acc[GW * GW / 256];
 #pragma unroll
   for (int k = 0; k < GW * GW / 256; k++) acc[k] = 0.0;
   for (int64_t r0 = r_begin; r0 < r_end; r0 += GR) {
-    stage(r0);
+    for (int e = tid; e < GR * GW; e += 256) {
+      const int rr = e % GR, cc = e / GR;
+      const int64_t r = r0 + rr;
+      sV[rr][cc] = (r < r_end && cc < mv) ? V[r + n * cc] : 0.0;
+      sW[rr][cc] = (r < r_end && cc < mw) ? W[r + n * cc] : 0.0;
+    }
+    __syncthreads();
 #pragma unroll
     for (int k = 0; k < GW * GW / 256; k++) {
       const int o = tid + 256 * k;
       if (o < cnt) {
         const int i = o % mv, j = o / mv;
         double a = acc[k];
-        for (int rr = 0; rr < GR; rr++) a += sV[i][rr] * sW[j][rr];
+        for (int rr = 0; rr < GR; rr++) a += sV[rr][i] * sW[rr][j];
         acc[k] = a;
       }
     }
@@ -406,7 +372,6 @@ void jacobi_eigh(int m, std::vector<double> &A, std::vector<double> &w, std::vec
 struct Dav {
   fcg_ctx *ctx = nullptr;
   int64_t n = 0;
-  int64_t crow = 0;  // rows per Gram chunk
   int nchunk = 0;
   double *V = nullptr, *W = nullptr, *X = nullptr, *AX = nullptr, *T = nullptr, *T2 = nullptr;
   double *hd = nullptr, *small = nullptr, *theta = nullptr, *part = nullptr;
@@ -439,12 +404,11 @@ int gram(Dav &d, const double *A, int ma, const double *B, int mb, double *dev_o
   if (ld <= 0) ld = ma;
   if (ma <= GW && mb <= GW) {
     hipLaunchKernelGGL(k_gram_partial_wide, dim3((unsigned)d.nchunk), dim3(256), 0, ctx->stream,
-                       d.n, A, ma, B, mb, d.crow, d.part);
+                       d.n, A, ma, B, mb, d.part);
   } else {
     const dim3 grid((unsigned)d.nchunk, (unsigned)((ma + GT - 1) / GT),
                     (unsigned)((mb + GT - 1) / GT));
-    hipLaunchKernelGGL(k_gram_partial, grid, dim3(256), 0, ctx->stream, d.n, A, ma, B, mb, d.crow,
-                       d.part);
+    hipLaunchKernelGGL(k_gram_partial, grid, dim3(256), 0, ctx->stream, d.n, A, ma, B, mb, d.part);
   }
   const int cnt = ma * mb;
   hipLaunchKernelGGL(k_gram_reduce, dim3((unsigned)cnt), dim3(64), 0, ctx->stream, d.nchunk, ma,
@@ -553,8 +517,7 @@ extern "C" int fcg_davidson(fcg_ctx_t ctx, fcg_plan_t pl, int R, const double *v
   d.ctx = ctx;
   const int64_t n = pl->sp->nvar;
   d.n = n;
-  d.crow = std::max<int64_t>(1, (n + 32 * GCHUNKS - 1) / (32 * GCHUNKS)) * 32;
-  d.nchunk = (int)((n + d.crow - 1) / d.crow);
+  d.nchunk = (int)((n + GCHUNK - 1) / GCHUNK);
   const int low = o->precision;
   if (low < FCG_FP64 || low >= FCG_N_PREC) {
     ctx->err = "unknown sigma precision";
