@@ -30,8 +30,9 @@
 
 namespace {
 
-constexpr int GT = 16;            // Gram output tile (GT x GT per workgroup)
-constexpr int GROWS = 64;         // rows staged in LDS per step
+constexpr int GT = 8;             // Gram output tile (GT x GT per workgroup)
+constexpr int GROWS = 128;        // rows staged in LDS per step
+constexpr int GTHR = 256;         // threads of a Gram workgroup
 constexpr int64_t GCHUNK = 4096;  // rows per split-K chunk
 constexpr int EMAX = 96;          // largest subspace whose eigenproblem runs on the GPU
 constexpr int ET = 1024;          // threads of the eigensolver workgroup
@@ -57,72 +58,103 @@ __global__ void k_precond(int64_t n, int R, const double *hd, const double *thet
   }
 }
 
-// part[chunk][i + mv*j] = sum over the chunk's rows of V[r,i] W[r,j]
-__global__ __launch_bounds__(256) void k_gram_partial(int64_t n, const double *V, int mv,
-                                                      const double *W, int mw, double *part) {
-  __shared__ double sV[GROWS][GT + 1];
-  __shared__ double sW[GROWS][GT + 1];
-  const int tid = threadIdx.x, ti = tid % GT, tj = tid / GT;
-  const int i0 = blockIdx.y * GT, j0 = blockIdx.z * GT;
-  const int64_t r_begin = (int64_t)blockIdx.x * GCHUNK;
-  const int64_t r_end = std::min<int64_t>(n, r_begin + GCHUNK);
-  double acc = 0.0;
-  for (int64_t r0 = r_begin; r0 < r_end; r0 += GROWS) {
-    for (int e = tid; e < GROWS * GT; e += 256) {
-      const int rr = e % GROWS, cc = e / GROWS;
-      const int64_t r = r0 + rr;
-      sV[rr][cc] = (r < r_end && i0 + cc < mv) ? V[r + n * (i0 + cc)] : 0.0;
-      sW[rr][cc] = (r < r_end && j0 + cc < mw) ? W[r + n * (j0 + cc)] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll 8
-    for (int rr = 0; rr < GROWS; rr++) acc += sV[rr][ti] * sW[rr][tj];
-    __syncthreads();
-  }
-  const int i = i0 + ti, j = j0 + tj;
-  if (i < mv && j < mw) part[(int64_t)blockIdx.x * mv * mw + i + (int64_t)mv * j] = acc;
-}
-
-// part[chunk][i + mv*j] as k_gram_partial, for mv, mw <= GW: one workgroup
-// per row chunk covers every output, so V and W are read once
-constexpr int GW = 64, GR = 32;
-__global__ __launch_bounds__(256) void k_gram_partial_wide(int64_t n, const double *V, int mv,
-                                                           const double *W, int mw,
-                                                           double *part) {
-  __shared__ double sV[GR][GW + 1];
-  __shared__ double sW[GR][GW + 1];
+// part[chunk][i + mv*j] = sum over the chunk's rows of V[r,i] W[r,j], each
+// output one chain of fused multiply-adds in row order (the order decides the
+// last bits, and with them the signs Davidson's vectors come out with).  What
+// bounds it at small n is that chain, 4,096 steps long however many
+// workgroups there are, so everything else is kept out of its way: a
+// workgroup owns 8 x 8 outputs, its first wavefront runs their chains from
+// LDS, two rows per 16-byte read, and all wavefronts load the next four
+// stages meanwhile.  At n = 9,125 (24 x 2 outputs) 224 us -> 28 us; one workgroup
+// per chunk with every output, 16 of them per thread, staged 64 columns
+// whether they existed or not and waited on LDS for each row.
+constexpr int GAHEAD = 4;  // stages loaded ahead
+static_assert(GAHEAD % 2 == 0, "stage d uses LDS buffer d & 1 in every round");
+constexpr int GB = 8;      // row pairs read from LDS at a time
+constexpr int GPAD = 2;  // doubles between staged columns: 16-byte aligned, banks spread
+__global__ __launch_bounds__(GTHR, 1) void k_gram_partial(int64_t n,
+                                                       const double *__restrict__ V,
+                                                       int mv, const double *__restrict__ W,
+                                                       int mw, double *__restrict__ part) {
+  __shared__ __align__(16) double sX[2][2 * GT][GROWS + GPAD];
   const int tid = threadIdx.x;
-  const int cnt = mv * mw;
+  const int i0 = blockIdx.y * GT, j0 = blockIdx.z * GT;
+  const int nv = min(GT, mv - i0), nw = min(GT, mw - j0);
   const int64_t r_begin = (int64_t)blockIdx.x * GCHUNK;
   const int64_t r_end = std::min<int64_t>(n, r_begin + GCHUNK);
-  double acc[GW * GW / 256];
+  // column slot cc of the stage: V's columns first, then W's; loads go to a
+  // clamped (valid) element and are masked when stored, so that they carry no
+  // branch and GAHEAD stages stay in flight
+  constexpr int PER = 2 * GT * GROWS / GTHR;
+  const int rr0 = tid % GROWS, cc0 = tid / GROWS;
+  const double *col[PER];
+  bool live[PER];
 #pragma unroll
-  for (int k = 0; k < GW * GW / 256; k++) acc[k] = 0.0;
-  for (int64_t r0 = r_begin; r0 < r_end; r0 += GR) {
-    for (int e = tid; e < GR * GW; e += 256) {
-      const int rr = e % GR, cc = e / GR;
-      const int64_t r = r0 + rr;
-      sV[rr][cc] = (r < r_end && cc < mv) ? V[r + n * cc] : 0.0;
-      sW[rr][cc] = (r < r_end && cc < mw) ? W[r + n * cc] : 0.0;
-    }
-    __syncthreads();
+  for (int k = 0; k < PER; k++) {
+    const int cc = cc0 + k * (GTHR / GROWS);
+    const bool isv = cc < GT;
+    const int c = isv ? cc : cc - GT, nc = isv ? nv : nw;
+    live[k] = c < nc;
+    col[k] = isv ? V + n * (i0 + min(c, nc - 1)) : W + n * (j0 + min(c, nc - 1));
+  }
+  double v[GAHEAD][PER];
+  auto load = [&](int64_t r0, double (&x)[PER]) {
+    const int64_t r = std::min<int64_t>(r0 + rr0, r_end - 1);
 #pragma unroll
-    for (int k = 0; k < GW * GW / 256; k++) {
-      const int o = tid + 256 * k;
-      if (o < cnt) {
-        const int i = o % mv, j = o / mv;
-        double a = acc[k];
-        for (int rr = 0; rr < GR; rr++) a += sV[rr][i] * sW[rr][j];
-        acc[k] = a;
+    for (int k = 0; k < PER; k++) x[k] = col[k][r];
+  };
+  auto store = [&](int64_t r0, const double (&x)[PER], int buf) {
+#pragma unroll
+    for (int k = 0; k < PER; k++)
+      sX[buf][cc0 + k * (GTHR / GROWS)][rr0] = live[k] && r0 + rr0 < r_end ? x[k] : 0.0;
+  };
+#pragma unroll
+  for (int d = 0; d < GAHEAD; d++) load(r_begin + d * GROWS, v[d]);
+  store(r_begin, v[0], 0);
+  load(r_begin + GAHEAD * GROWS, v[0]);
+  __syncthreads();
+  const int i = tid % GT, j = (tid / GT) % GT;
+  double acc = 0.0;
+  for (int64_t r0 = r_begin; r0 < r_end; r0 += GAHEAD * GROWS) {
+#pragma unroll
+    for (int d = 0; d < GAHEAD; d++) {
+      const int buf = d & 1;
+      if (tid < GT * GT) {
+        const double2 *a = reinterpret_cast<const double2 *>(sX[buf][i]);
+        const double2 *b = reinterpret_cast<const double2 *>(sX[buf][GT + j]);
+        // eight row pairs read ahead of the eight in use: left to itself the
+        // compiler reads each pair where it is used and waits for LDS
+        double2 x[2][GB], y[2][GB];
+        auto fetch = [&](int p, double2 (&u)[GB], double2 (&w)[GB]) {
+#pragma unroll
+          for (int k = 0; k < GB; k++) {
+            u[k] = a[p + k];
+            w[k] = b[p + k];
+          }
+        };
+        fetch(0, x[0], y[0]);
+#pragma unroll
+        for (int p = 0; p < GROWS / 2; p += GB) {
+          const int h = (p / GB) & 1;
+          if (p + GB < GROWS / 2) fetch(p + GB, x[h ^ 1], y[h ^ 1]);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int k = 0; k < GB; k++) {
+            acc += x[h][k].x * y[h][k].x;
+            acc += x[h][k].y * y[h][k].y;
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
+      // rows past the chunk's end are staged as zeros
+      const int64_t nx = r0 + (d + 1) * GROWS;
+      store(nx, v[(d + 1) % GAHEAD], buf ^ 1);
+      load(nx + GAHEAD * GROWS, v[(d + 1) % GAHEAD]);
+      __syncthreads();
     }
-    __syncthreads();
   }
-#pragma unroll
-  for (int k = 0; k < GW * GW / 256; k++) {
-    const int o = tid + 256 * k;
-    if (o < cnt) part[(int64_t)blockIdx.x * cnt + o] = acc[k];
-  }
+  if (tid < GT * GT && i < nv && j < nw)
+    part[(int64_t)blockIdx.x * mv * mw + (i0 + i) + (int64_t)mv * (j0 + j)] = acc;
 }
 
 // out[i + ld*j] = sum over chunks of part[chunk][i + ma*j], one wavefront per
@@ -402,14 +434,9 @@ int gram(Dav &d, const double *A, int ma, const double *B, int mb, double *dev_o
          std::vector<double> *host_out, int ld = 0) {
   fcg_ctx *ctx = d.ctx;
   if (ld <= 0) ld = ma;
-  if (ma <= GW && mb <= GW) {
-    hipLaunchKernelGGL(k_gram_partial_wide, dim3((unsigned)d.nchunk), dim3(256), 0, ctx->stream,
-                       d.n, A, ma, B, mb, d.part);
-  } else {
-    const dim3 grid((unsigned)d.nchunk, (unsigned)((ma + GT - 1) / GT),
-                    (unsigned)((mb + GT - 1) / GT));
-    hipLaunchKernelGGL(k_gram_partial, grid, dim3(256), 0, ctx->stream, d.n, A, ma, B, mb, d.part);
-  }
+  const dim3 grid((unsigned)d.nchunk, (unsigned)((ma + GT - 1) / GT),
+                  (unsigned)((mb + GT - 1) / GT));
+  hipLaunchKernelGGL(k_gram_partial, grid, dim3(GTHR), 0, ctx->stream, d.n, A, ma, B, mb, d.part);
   const int cnt = ma * mb;
   hipLaunchKernelGGL(k_gram_reduce, dim3((unsigned)cnt), dim3(64), 0, ctx->stream, d.nchunk, ma,
                      cnt, d.part, dev_out, ld);

@@ -1,0 +1,55 @@
+"""Davidson where its tall-skinny products have edges: spaces around a stage
+of rows (128) and the rounds of stages, root counts below, at and above an
+output tile (8 columns), and subspaces above the GPU eigensolver's limit.
+
+Reference: the eigenvalues and residuals of the dense H of the same space
+(build_full_H, symmetrised).  Bars: the solver stops at a residual norm of
+1e-9, so each energy lies within 1e-9 of an eigenvalue of H, and the residual
+recomputed here within 2e-9 (its own rounding is 1e-13); orthonormal vectors to
+1e-11 (two Gram-Schmidt rounds, at most 256 columns).
+"""
+import numpy as np
+import pytest
+
+from fermicg_amd.state import TPSCIstate
+from fermicg_amd.tpsci import Engine, build_full_H
+from fermicg_amd.workloads import tpsci_small
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def problem():
+    p, st = tpsci_small(seed=3)
+    return p, st, Engine(0)
+
+
+def _subspace(st, n):
+    """The first n configurations."""
+    f = int(np.searchsorted(st.fock_start, n, side="left"))
+    s = TPSCIstate(st.N, 1)
+    s.fock, s.cfg = st.fock[:f], st.cfg[:n]
+    s.fock_start = np.minimum(st.fock_start[:f + 1], n)
+    s.coeffs = np.zeros((n, 1))
+    return s
+
+
+@pytest.mark.parametrize("n,R,ss", [(31, 1, 12), (127, 2, 8), (129, 3, 4), (512, 1, 24), (513, 2, 30),
+                                    (513, 6, 8), (640, 9, 6), (1500, 16, 5)])
+def test_davidson_sizes(problem, n, R, ss):
+    p, st, eng = problem
+    sub = _subspace(st, n)
+    H = build_full_H(sub, p.cluster_ops, p.clustered_ham, engine=eng)
+    H = 0.5 * (H + H.T)
+    order = np.argsort(np.diag(H))
+    v0 = np.zeros((n, R))
+    v0[order[:R], np.arange(R)] = 1.0
+    v0 += 0.01 * np.random.Generator(np.random.PCG64(n)).normal(size=(n, R))
+    pl = eng.tpsci_plan(sub, p.cluster_ops, p.clustered_ham)
+    e, v, stats = pl.davidson(v0, conv_thresh=1e-9, max_iter=500, max_ss_vecs=ss)
+    print("n", n, "R", R, stats["iterations"], stats["converged"], flush=True)
+    assert stats["converged"]
+    w = np.linalg.eigvalsh(H)
+    assert max(np.abs(w - x).min() for x in e) < 1e-9
+    assert np.linalg.norm(H @ v - v * e, axis=0).max() < 2e-9
+    assert np.abs(v.T @ v - np.eye(R)).max() < 1e-11
