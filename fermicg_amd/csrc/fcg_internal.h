@@ -38,6 +38,29 @@ constexpr int FCG_MAX_R = 16;         // roots per sigma launch
 constexpr int FCG_N_PREC = 5;  // FCG_FP64 .. FCG_FP32_BF16C
 constexpr int FCG_QUAD = 4;           // panel columns per stored column quad
 constexpr int FCG_CSR_WPB = 4;        // one-row boxes: wavefronts (rows) per workgroup
+// Plans with fewer multi-row boxes than this share each panel of at least
+// FCG_SHARE_MIN elements between the wavefronts of a workgroup
+// (k_apply_stream); with more, one wavefront per box (k_apply) already fills
+// the chip and wastes less on short panels.  Measured, shared against not:
+// 73 boxes FP64 58 / 110 us; 2,380 boxes FP32 288 / 541 us; 9,408 boxes FP64
+// 1.95 / 2.83 ms; 28,784 boxes FP64 10.1 / 10.2 ms but FP32 6.5 / 5.5 ms.
+// Sharing only the largest panels leaves two launches, each with its own
+// tail: 28,784 boxes FP32 5.8-6.4 ms.
+constexpr int64_t FCG_SHARE_BOXES = 16384, FCG_SHARE_MIN = 8192;
+// Row groups (workgroups) per shared panel: enough for two workgroups per CU,
+// at most eight of a 64-row panel (a group's rows then read 128-byte runs of
+// FP32).  73 panels of 64 rows, FP64: 69 us in four groups, 58 in eight.
+inline int fcg_split_parts(int64_t n_split) {
+  int p = 1;
+  while (p < 8 && n_split > 0 && n_split * p < 512) p *= 2;
+  return p;
+}
+// Plans with fewer one-row boxes than this share each between this many
+// wavefronts (FP64 sums only: FP32 ones keep the order, and so the rounding,
+// of a wavefront per row).  661 rows of 10,000 columns: 128 us with a
+// wavefront each, 20 shared.
+constexpr int64_t FCG_SHARED_ROWS = 2048;
+constexpr int FCG_ROW_WAVES = 8;
 constexpr int FCG_XCDS = 8;           // MI355X accelerator complex dies (workgroups round-robin)
 
 // Row panel storage.  The Hamiltonian blocks of one bra box (db rows) sit
@@ -173,6 +196,9 @@ struct fcg_plan {
   // that each XCD's workgroups take a contiguous run of rows
   int32_t *d_order = nullptr;
   int64_t n_multi = 0, n_single_slots = 0;
+  int64_t n_split = 0;   // the first boxes of the order, applied by k_apply_stream
+  int split_parts = 1;   // ... in this many row groups each (fcg_split_parts)
+  int64_t n_single = 0;  // one-row boxes
   int32_t *d_colidx = nullptr;    // [n_cols] column -> variable index
   int64_t n_cols = 0;
   double *d_K64 = nullptr;
@@ -240,7 +266,7 @@ struct HostPlan {
   RawVec<int64_t> pair_t0, pair_koff;
   std::vector<int64_t> row_ptr, diag_koff, row_koff, col_ptr;
   std::vector<int32_t> diag_col, order;
-  int64_t n_multi = 0, n_single_slots = 0;
+  int64_t n_multi = 0, n_single_slots = 0, n_split = 0, n_single = 0;
   RawVec<TaskDev> tasks;
   // pair indices for the block build: pairs within the tiny class's limits
   // first (n_tiny of them; plans that store their blocks only), then those
@@ -254,7 +280,8 @@ struct HostPlan {
 };
 // apply schedule of a plan (see fcg_plan::d_order)
 void fcg_apply_order(const std::vector<int64_t> &var_off, const std::vector<int64_t> &col_ptr,
-                     std::vector<int32_t> *order, int64_t *n_multi, int64_t *n_single_slots);
+                     std::vector<int32_t> *order, int64_t *n_multi, int64_t *n_single_slots,
+                     int64_t *n_split, int64_t *n_single);
 // layout = false: pairs, tasks and LDS classes only (a plan whose blocks are
 // used once during the build); pair_col, pair_koff, the row panels, colidx,
 // the apply order and the diagonal tables are left empty

@@ -713,6 +713,217 @@ __global__ __launch_bounds__(64 * WPB) void k_apply(int64_t n_box,
   }
 }
 
+// The larger panels of a plan (fcg_plan::n_split): one workgroup per bra box
+// (or per group of its rows, `parts` groups) streams the panel through LDS.
+// The sums are k_apply's, term by term: row i's slice s takes the quads j of
+// each CG-quad chunk with (j mod CG) mod sl == s in order, and the slices are
+// added in order -- only the loads are shared, by all four wavefronts, a
+// stage of SB bytes ahead of the one in use, so a panel's bandwidth no longer
+// depends on one wavefront's registers (about 6 GB/s).  Bound by HBM; a
+// (row, slice, root) chain costs four dependent multiply-adds per quad, which
+// is why the roots go to different wavefronts and LDS is read a batch ahead.
+template <typename TK, typename TA, typename TC, int R, int SB, bool NT>
+__global__ __launch_bounds__(256) void k_apply_stream(
+    int parts, const int32_t *__restrict__ order, const int64_t *__restrict__ var,
+    const int64_t *__restrict__ row_koff, const int64_t *__restrict__ col_ptr,
+    const int32_t *__restrict__ colidx, const TK *__restrict__ K, const TC *__restrict__ c,
+    int64_t nvar_s, double *__restrict__ sigma) {
+  constexpr int CG = stage_quads<TC, R>();
+  constexpr int QB = FCG_QUAD * (int)sizeof(TK);  // bytes of a quad's row
+  constexpr int LU = QB < 16 ? QB : 16;           // bytes per load
+  constexpr int NU = SB / LU / 256;               // loads per thread and stage
+  constexpr int TR = R < 4 ? R : 4;               // root lanes (wavefronts)
+  constexpr int RPT = (R + TR - 1) / TR;          // roots per thread
+  // quads read from LDS at a time: at most 12 reads, which the 4-bit LDS
+  // counter can still tell from the batch before (16 made each batch wait)
+  constexpr int LPQ = (QB + 15) / 16 + RPT * (int)sizeof(TC) / 4;
+  constexpr int UQ = LPQ > 12 ? 1 : 12 / LPQ;
+  // stages in flight, held in registers until their turn: as many as leave
+  // room for two workgroups per CU
+  constexpr int D = R * (int)sizeof(TC) <= 16 ? 4 : 2;
+  static_assert(4 * CG <= 256 && SB >= FCG_MAX_BOX * QB && SB % (256 * LU) == 0, "stage shape");
+  using Unit = std::conditional_t<LU == 16, nu4, nu2>;
+  __shared__ __align__(16) Unit sK[2][SB / LU];
+  __shared__ __align__(16) TC sC[2][CG * R * FCG_QUAD];
+  __shared__ TA sRed[R][64];
+  const int tid = threadIdx.x;
+  const int64_t b = order[blockIdx.x / parts];
+  const int64_t v0 = var[b];
+  const int db = (int)(var[b + 1] - v0);
+  const int rpw = (db + parts - 1) / parts;
+  const int r0 = rpw * (int)(blockIdx.x % parts);
+  const int dr = min(rpw, db - r0);
+  if (dr <= 0) return;  // uniform: fewer rows than groups
+  const int sl = 64 / db;
+  const int64_t c0 = col_ptr[b];
+  const int ngrp = (int)((col_ptr[b + 1] - c0) / FCG_QUAD);
+  const int32_t *ci = colidx + c0;
+  const char *Kp = reinterpret_cast<const char *>(K + row_koff[b]) + r0 * QB;
+  const int Q = min(CG, SB / (dr * QB));  // quads per stage
+  const int w = dr * QB / LU;             // loads per quad
+  // stages: [base + o, base + o + Q) within the chunk [base, base + CG)
+  struct At { int base, o; };
+  auto next = [&](At x) {
+    x.o += Q;
+    if (x.o >= CG || x.base + x.o >= ngrp) return At{x.base + CG, 0};
+    return x;
+  };
+  auto quads = [&](At x) { return min(min(Q, CG - x.o), ngrp - x.base - x.o); };
+  // loads are unconditional, from clamped (valid) places, so that they carry
+  // no branch and each wait is for its own stage only
+  Unit kr[D][NU];
+  TC cr[D][R];
+  int idx[D];
+  const int utop = Q * w - 1;
+  int uq[NU];          // this thread's loads: quad of the stage
+  int64_t uo[NU];      // ... and byte offset from the quad
+#pragma unroll
+  for (int k = 0; k < NU; k++) {
+    const int e = min(tid + 256 * k, utop);
+    uq[k] = e / w;
+    uo[k] = e % w * LU;
+  }
+  auto load_idx = [&](At x, int d) {
+    idx[d] = ci[min(FCG_QUAD * (x.base + x.o) + min(tid, FCG_QUAD * Q - 1), FCG_QUAD * ngrp - 1)];
+  };
+  auto load = [&](At x, int d) {
+    load_row<TC, R>(c + (int64_t)idx[d] * R, cr[d]);
+#pragma unroll
+    for (int k = 0; k < NU; k++) {
+      const int q = min(x.base + x.o + uq[k], ngrp - 1);
+      kr[d][k] = ld_stream<NT>(reinterpret_cast<const Unit *>(Kp + (int64_t)q * db * QB + uo[k]));
+    }
+  };
+  auto store = [&](int d, int buf) {
+#pragma unroll
+    for (int k = 0; k < NU; k++)
+      if (tid + 256 * k <= utop) sK[buf][tid + 256 * k] = kr[d][k];
+    if (tid < FCG_QUAD * Q) {
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        sC[buf][((tid >> 2) * R + r) * FCG_QUAD + (tid & 3)] = cr[d][r];
+    }
+  };
+  // the wavefronts that run chains differ between neighbouring workgroups, so
+  // that a CU's chains do not share one SIMD
+  const int tr = ((tid >> 6) + (int)(blockIdx.x / FCG_XCDS)) & 3, p = tid & 63;
+  const int i = p % dr, s = p / dr;
+  const bool act = s < sl && tr < TR;
+  TA acc[RPT];
+#pragma unroll
+  for (int m = 0; m < RPT; m++) acc[m] = (TA)0;
+  if (ngrp > 0) {
+    At cur{0, 0}, ahead{0, 0};  // the stage in use, the next stage to load
+    At aidx{0, 0};              // the next stage whose column indices to load
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      load_idx(aidx, d);
+      aidx = next(aidx);
+    }
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      load(ahead, d);
+      ahead = next(ahead);
+      load_idx(aidx, d);
+      aidx = next(aidx);
+    }
+    store(0, 0);
+    load(ahead, 0);
+    ahead = next(ahead);
+    load_idx(aidx, 0);
+    aidx = next(aidx);
+    __syncthreads();
+    while (cur.base < ngrp) {
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        const int buf = d & 1;
+        if (act && cur.base < ngrp) {
+          const int qn = quads(cur);
+          const int om = cur.o % sl;
+          const int f = s >= om ? s - om : s - om + sl;  // first quad of this slice
+          const int nq = f < qn ? (qn - f + sl - 1) / sl : 0;
+          const char *kb = reinterpret_cast<const char *>(sK[buf]) + i * QB;
+          const TC *cb = sC[buf];
+          // whole batches of UQ quads, the next one read while one is used: the
+          // chains run on one wavefront, so every instruction in here counts
+          // (pointers step by constants, no clamps); then the rest one by one
+          const char *kp = kb + f * dr * QB;
+          const TC *cp = cb + f * R * FCG_QUAD;
+          const int ks = sl * dr * QB, cs = sl * R * FCG_QUAD;
+          RawQuad<TK> kv[2][UQ];
+          TC cv[2][UQ][RPT][FCG_QUAD];
+          auto fetch = [&](RawQuad<TK> &kk, TC (&cc)[RPT][FCG_QUAD]) {
+            kk.template load<false>(reinterpret_cast<const TK *>(kp));
+  #pragma unroll
+            for (int m = 0; m < RPT; m++) {
+              const int r = RPT * TR == R ? tr + TR * m : min(tr + TR * m, R - 1);
+              stage_read<TC, FCG_QUAD>(cp + r * FCG_QUAD, cc[m]);
+            }
+            kp += ks;
+            cp += cs;
+          };
+          auto use = [&](const RawQuad<TK> &kk, const TC (&cc)[RPT][FCG_QUAD]) {
+            TA kq[FCG_QUAD];
+            kk.get(kq);
+  #pragma unroll
+            for (int q = 0; q < FCG_QUAD; q++)
+  #pragma unroll
+              for (int m = 0; m < RPT; m++) acc[m] += kq[q] * (TA)cc[m][q];
+          };
+          auto fetch_batch = [&](int h) {
+  #pragma unroll
+            for (int u = 0; u < UQ; u++) fetch(kv[h][u], cv[h][u]);
+            __builtin_amdgcn_sched_barrier(0);
+          };
+          auto use_batch = [&](int h) {
+  #pragma unroll
+            for (int u = 0; u < UQ; u++) use(kv[h][u], cv[h][u]);
+            __builtin_amdgcn_sched_barrier(0);
+          };
+          int left = nq / UQ;
+          if (left > 0) {
+            fetch_batch(0);
+            for (; left > 2; left -= 2) {
+              fetch_batch(1);
+              use_batch(0);
+              fetch_batch(0);
+              use_batch(1);
+            }
+            if (left == 2) {
+              fetch_batch(1);
+              use_batch(0);
+              use_batch(1);
+            } else {
+              use_batch(0);
+            }
+          }
+          for (int n = nq % UQ; n > 0; n--) {
+            fetch(kv[0][0], cv[0][0]);
+            use(kv[0][0], cv[0][0]);
+          }
+        }
+        store((d + 1) % D, buf ^ 1);
+        load(ahead, (d + 1) % D);
+        ahead = next(ahead);
+        load_idx(aidx, (d + 1) % D);
+        aidx = next(aidx);
+        __syncthreads();
+        cur = next(cur);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < RPT; m++)
+    if (tr < TR && tr + TR * m < R) sRed[tr + TR * m][p] = act ? acc[m] : (TA)0;
+  __syncthreads();
+  for (int e = tid; e < dr * R; e += 256) {
+    const int row = e % dr, r = e / dr;
+    TA v = (TA)0;
+    for (int s2 = 0; s2 < sl; s2++) v += sRed[r][row + dr * s2];
+    sigma[(int64_t)r * nvar_s + v0 + r0 + row] = (double)v;
+  }
+}
+
 // One-row boxes (db = 1, the rows of sparse TPSCI spaces): no row shares a
 // column with another, so there is nothing to stage; the wave streams the
 // row's columns in slabs of 64*4U, lane l taking columns l, l+64, ... of a
@@ -722,16 +933,20 @@ __global__ __launch_bounds__(64 * WPB) void k_apply(int64_t n_box,
 // instruction (1.45x over quad-per-lane gathers on the 2e6-configuration
 // rank-1 space).  Rows come from `order` (XCD-grouped slots, -1 = empty);
 // the 64 lane sums are combined by a fixed butterfly.
-template <typename TK, typename TA, typename TC, int R, int U, bool NT>
-__global__ __launch_bounds__(64 * FCG_CSR_WPB) void k_apply_rows(
+// WPR = 1: a workgroup's wavefronts take a row each.  WPR > 1: they
+// share one row, a contiguous part each, summed in order -- for plans with
+// fewer rows than the chip holds wavefronts (FCG_SHARED_ROWS).
+template <typename TK, typename TA, typename TC, int R, int U, bool NT, int WPR>
+__global__ __launch_bounds__(64 * (WPR > 1 ? WPR : FCG_CSR_WPB)) void k_apply_rows(
     int64_t n_slots, const int32_t *__restrict__ order, const int64_t *__restrict__ var,
     const int64_t *__restrict__ row_koff, const int64_t *__restrict__ col_ptr,
     const int32_t *__restrict__ colidx, const TK *__restrict__ K, const TC *__restrict__ c,
     int64_t nvar_s, double *__restrict__ sigma) {
+  __shared__ TA sPart[WPR][R];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t w = (int64_t)blockIdx.x * FCG_CSR_WPB + wave;
+  const int64_t w = WPR > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * FCG_CSR_WPB + wave;
   const int32_t b = w < n_slots ? order[w] : -1;
-  if (b < 0) return;  // uniform per wave
+  if (b < 0) return;  // uniform per wave (and per workgroup when it shares a row)
   const int64_t c0 = col_ptr[b];
   const int ngrp = (int)((col_ptr[b + 1] - c0) / FCG_QUAD);
   const TK *Kr = K + row_koff[b];
@@ -739,11 +954,16 @@ __global__ __launch_bounds__(64 * FCG_CSR_WPB) void k_apply_rows(
   TA acc[R];
 #pragma unroll
   for (int r = 0; r < R; r++) acc[r] = (TA)0;
-  const int ncol = FCG_QUAD * ngrp;
+  int first = 0, ncol = FCG_QUAD * ngrp;
+  if (WPR > 1) {
+    const int per = (ncol + 64 * WPR - 1) / (64 * WPR) * 64;
+    first = per * wave;
+    ncol = min(ncol, first + per);
+  }
   const TK *Kl = Kr + lane;
   const int32_t *cl = ci + lane;
   constexpr int NE = 4 * U;  // columns in flight per lane
-  for (int s0 = 0; s0 < ncol; s0 += 64 * NE) {
+  for (int s0 = first; s0 < ncol; s0 += 64 * NE) {
     TK kv[NE];
     int idx[NE];
 #pragma unroll
@@ -773,7 +993,18 @@ __global__ __launch_bounds__(64 * FCG_CSR_WPB) void k_apply_rows(
     for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
     acc[r] = v;
   }
-  if (lane == 0) {
+  if (WPR > 1) {
+    if (lane == 0) {
+#pragma unroll
+      for (int r = 0; r < R; r++) sPart[wave][r] = acc[r];
+    }
+    __syncthreads();
+    if (threadIdx.x < R) {
+      TA v = (TA)0;
+      for (int k = 0; k < WPR; k++) v += sPart[k][threadIdx.x];
+      sigma[(int64_t)threadIdx.x * nvar_s + var[b]] = (double)v;
+    }
+  } else if (lane == 0) {
 #pragma unroll
     for (int r = 0; r < R; r++) sigma[(int64_t)r * nvar_s + var[b]] = (double)acc[r];
   }
@@ -939,18 +1170,39 @@ template <typename TK, typename TA, typename TC, int R, int V>
 void launch_multi_v(const fcg_plan *pl, const TK *K, const TC *c, double *sigma, hipStream_t s) {
   constexpr int W = kMulti[V].wpb, U = kMulti[V].unroll;
   constexpr bool NT = kMulti[V].nt;
-  hipLaunchKernelGGL((k_apply<TK, TA, TC, R, W, U, apply_clamp<TK>(), NT>),
-                     dim3((unsigned)((pl->n_multi + W - 1) / W)), dim3(64 * W), 0, s, pl->n_multi,
-                     pl->d_order, pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr, pl->d_colidx, K, c,
-                     pl->sp->nvar, sigma);
+  const int64_t ns = pl->n_split, n1 = pl->n_multi - ns;
+  if (ns > 0) {
+    constexpr int SB = (U >= 16 ? 16384 : 8192) / (sizeof(TK) == 2 ? 2 : 1);
+    hipLaunchKernelGGL((k_apply_stream<TK, TA, TC, R, SB, NT>),
+                       dim3((unsigned)(ns * pl->split_parts)), dim3(256), 0, s, pl->split_parts,
+                       pl->d_order, pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr, pl->d_colidx, K,
+                       c, pl->sp->nvar, sigma);
+  }
+  if (n1 > 0)
+    hipLaunchKernelGGL((k_apply<TK, TA, TC, R, W, U, apply_clamp<TK>(), NT>),
+                       dim3((unsigned)((n1 + W - 1) / W)), dim3(64 * W), 0, s, n1,
+                       pl->d_order + ns, pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr,
+                       pl->d_colidx, K, c, pl->sp->nvar, sigma);
 }
 
 template <typename TK, typename TA, typename TC, int R, int V>
 void launch_rows_v(const fcg_plan *pl, const TK *K, const TC *c, double *sigma, hipStream_t s) {
-  hipLaunchKernelGGL((k_apply_rows<TK, TA, TC, R, kRows[V].unroll, kRows[V].nt>),
-                     dim3((unsigned)(pl->n_single_slots / FCG_CSR_WPB)), dim3(64 * FCG_CSR_WPB), 0,
-                     s, pl->n_single_slots, pl->d_order + pl->n_multi, pl->sp->d_var,
-                     pl->d_row_koff, pl->d_col_ptr, pl->d_colidx, K, c, pl->sp->nvar, sigma);
+  auto launch = [&](auto wpr) {
+    constexpr int W = decltype(wpr)::value;
+    const int64_t n = pl->n_single_slots;
+    hipLaunchKernelGGL((k_apply_rows<TK, TA, TC, R, kRows[V].unroll, kRows[V].nt, W>),
+                       dim3((unsigned)(W > 1 ? n : n / FCG_CSR_WPB)),
+                       dim3(64 * (W > 1 ? W : FCG_CSR_WPB)), 0, s, n, pl->d_order + pl->n_multi,
+                       pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr, pl->d_colidx, K, c,
+                       pl->sp->nvar, sigma);
+  };
+  if constexpr (sizeof(TA) == 8) {
+    if (pl->n_single < FCG_SHARED_ROWS) {
+      launch(std::integral_constant<int, FCG_ROW_WAVES>{});
+      return;
+    }
+  }
+  launch(std::integral_constant<int, 1>{});
 }
 
 // parts: bit 0 multi-row boxes, bit 1 one-row boxes
@@ -1017,8 +1269,11 @@ hipError_t fcg_launch_apply(const fcg_plan *pl, int R, const double *c, double *
   }
   const int64_t nk = pl->ksp->nvar;
   if (precision == FCG_FP64) {
-    double *ci = static_cast<double *>(ci_buf);
-    hipLaunchKernelGGL(k_interleave<double>, dim3(1024), dim3(256), 0, s, nk, R, c, ci);
+    // one FP64 vector is its own interleaved copy
+    const double *ci = R == 1 ? c : static_cast<const double *>(ci_buf);
+    if (R > 1)
+      hipLaunchKernelGGL(k_interleave<double>, dim3(1024), dim3(256), 0, s, nk, R, c,
+                         static_cast<double *>(ci_buf));
     if (before_apply) (void)hipEventRecord(before_apply, s);
     return launch_by_r<double, double, double>(pl, R, vm, vr, parts, pl->d_K64, ci, sigma, s);
   }

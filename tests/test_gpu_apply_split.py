@@ -1,0 +1,63 @@
+"""The sigma apply where panels and rows are shared between wavefronts: boxes
+of 1 to 64 rows (dimensions that do and do not divide a wavefront), column
+counts that leave the last wavefronts little or nothing, and every root count
+with its own compiled form.
+
+Oracle: the C restatements of tps_ci_matvec and build_sigma!.  Bars as for the
+other sigma tests, relative to the largest element: FP64 1e-12, FP32 and split
+BF16 1e-5 and 1e-4, BF16 and a bf16 c 1e-2 (2e-3 per rounded factor).
+"""
+import numpy as np
+import pytest
+
+from fermicg_amd.bst import bst_pq_state, cache_hamiltonian
+from fermicg_amd.marshal import flatten_ham, flatten_ops
+from fermicg_amd.state import TPSCIstate
+from fermicg_amd.tpsci import Engine, cluster_sizes_of
+from fermicg_amd.workloads import build_problem
+from oracle.pyoracle import BstOracle, Oracle
+
+pytestmark = pytest.mark.gpu
+
+TOL = {"fp64": 1e-12, "fp32": 1e-5, "bf16x2": 1e-4, "bf16": 1e-2, "fp32_bf16c": 1e-2}
+
+
+@pytest.fixture(scope="module")
+def eng():
+    return Engine(0)
+
+
+def _check(plan, ref, c, label):
+    for prec, tol in TOL.items():
+        s = plan.sigma(c, prec)
+        err = np.abs(s - ref).max() / np.abs(ref).max()
+        print(label, prec, "%.2e" % err, flush=True)
+        assert err < tol
+
+
+@pytest.mark.parametrize("clusters,M,transfer,R", [(2, 3, 1, 1), (2, 7, 2, 3), (3, 3, 2, 2),
+                                                   (3, 4, 1, 4), (3, 5, 2, 1), (3, 4, 2, 5),
+                                                   (3, 4, 2, 16)])
+def test_full_blocks(eng, clusters, M, transfer, R):
+    p = build_problem(4 * clusters, clusters, M, 8 * clusters, seed=M, max_transfer=transfer)
+    st = TPSCIstate.full_blocks(p.bases, p.focks, R=R)
+    c = np.random.Generator(np.random.PCG64(R)).normal(size=(len(st), R))
+    st.set_vector(c)
+    ref = Oracle(flatten_ops(p.cluster_ops, cluster_sizes_of(p.cluster_ops)),
+                 flatten_ham(p.clustered_ham), st).sigma(c)
+    plan = eng.tpsci_plan(st, p.cluster_ops, p.clustered_ham, precisions=tuple(TOL))
+    _check(plan, ref, c, (clusters, M, transfer, R))
+    eng.drop_plans()
+
+
+@pytest.mark.parametrize("clusters,M,rank,R", [(2, 6, 5, 1), (3, 9, 8, 2), (3, 7, 6, 4), (3, 5, 3, 7)])
+def test_tucker_boxes(eng, clusters, M, rank, R):
+    p = build_problem(4 * clusters, clusters, M, 8 * clusters, seed=M, max_transfer=2)
+    st = bst_pq_state(p.bases, p.focks, p.ref_fock, max_rank=rank, R=R, seed=rank)
+    ref = BstOracle(flatten_ops(p.cluster_ops, cluster_sizes_of(p.cluster_ops)),
+                    flatten_ham(p.clustered_ham), st).sigma_rows(st.coeffs,
+                                                                np.arange(len(st.blocks)))[0]
+    plan = cache_hamiltonian(st, st, p.cluster_ops, p.clustered_ham, precisions=tuple(TOL),
+                             engine=eng)
+    _check(plan, ref, st.coeffs, (clusters, M, rank, R))
+    eng.drop_plans()
