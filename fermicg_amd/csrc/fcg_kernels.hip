@@ -1269,9 +1269,10 @@ hipError_t fcg_launch_apply(const fcg_plan *pl, int R, const double *c, double *
   }
   const int64_t nk = pl->ksp->nvar;
   if (precision == FCG_FP64) {
-    // one FP64 vector is its own interleaved copy
-    const double *ci = R == 1 ? c : static_cast<const double *>(ci_buf);
-    if (R > 1)
+    // one FP64 vector is its own interleaved copy, unless sigma overwrites it
+    const bool own = R == 1 && (c + nk <= sigma || sigma + sp->nvar <= c);
+    const double *ci = own ? c : static_cast<const double *>(ci_buf);
+    if (!own)
       hipLaunchKernelGGL(k_interleave<double>, dim3(1024), dim3(256), 0, s, nk, R, c,
                          static_cast<double *>(ci_buf));
     if (before_apply) (void)hipEventRecord(before_apply, s);

@@ -9,6 +9,7 @@ BF16 1e-5 and 1e-4, BF16 and a bf16 c 1e-2 (2e-3 per rounded factor).
 """
 import numpy as np
 import pytest
+import torch
 
 from fermicg_amd.bst import bst_pq_state, cache_hamiltonian
 from fermicg_amd.marshal import flatten_ham, flatten_ops
@@ -60,4 +61,23 @@ def test_tucker_boxes(eng, clusters, M, rank, R):
     plan = cache_hamiltonian(st, st, p.cluster_ops, p.clustered_ham, precisions=tuple(TOL),
                              engine=eng)
     _check(plan, ref, st.coeffs, (clusters, M, rank, R))
+    eng.drop_plans()
+
+
+@pytest.mark.parametrize("shift", [0, 1, 5])
+def test_sigma_over_its_vector(eng, shift):
+    """sigma_device with sigma over c, or overlapping it, gives what separate
+    buffers give (one FP64 vector, the case that is applied without a copy)."""
+    p = build_problem(12, 3, 4, 24, seed=4, max_transfer=1)
+    st = TPSCIstate.full_blocks(p.bases, p.focks, R=1)
+    n = len(st)
+    c = np.random.Generator(np.random.PCG64(1)).normal(size=(n, 1))
+    plan = eng.tpsci_plan(st, p.cluster_ops, p.clustered_ham)
+    ref = plan.sigma(c)[:, 0]
+    buf = torch.zeros(n + 8, dtype=torch.float64, device="cuda:0")
+    buf[shift:shift + n] = torch.from_numpy(c[:, 0]).to("cuda:0")
+    torch.cuda.synchronize()
+    plan.sigma_device(buf[shift:].data_ptr(), buf.data_ptr(), 1)
+    eng.ctx.synchronize()
+    assert np.array_equal(buf[:n].cpu().numpy(), ref)
     eng.drop_plans()
