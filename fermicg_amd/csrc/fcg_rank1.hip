@@ -100,289 +100,326 @@ struct R1Args {
   unsigned int *err;
 };
 
-// decode column-major index v over nb dims into p[0..nb)
-__device__ __forceinline__ void decode(int v, int nb, const int32_t *dims, int *p) {
-  for (int q = 0; q < nb; q++) {
-    p[q] = v % dims[q];
-    v /= dims[q];
-  }
-}
+constexpr int RP = 64;      // connected ket blocks looked up at a time
+constexpr int TS = 32;      // terms of a pair prepared at a time
+constexpr int NPS = 80;     // index values of a term's clusters together, and W_ab entries of
+constexpr int WABX = 768;   // its cluster pairs: at most 76 and 600 where every index count is
+                            // <= NPX, every pair's product <= 256 and the whole <= VMX
+constexpr int WIJ = 1024;   // staged w_ij values
 
+// a term prepared for the pair in hand
+struct R1Ready {
+  int64_t goff[4], ioff;
+  int32_t nb, nv, ok;
+  float sgn;
+  int16_t cl[4], np[4], mb[4], mk[4], poff[4];  // poff: first place among the NPS index values
+};
+
+// One workgroup per bra Fock block.  Per connected ket block and term the
+// work is a few thousand multiply-adds on small arrays, so what bounds it is
+// the number of dependent steps -- global round trips and barriers -- and
+// serial loops on few threads.  Hence: ket blocks are looked up RP at a time
+// and a pair's terms prepared TS at a time by one thread per (term, cluster);
+// W_a and e come from W_ab instead of from V again; the cross part W_ab u_b is
+// formed once per (a, p) instead of once per state of a; and the state
+// blocks' w_ij = W_a . Γ_a[:, i, j] are spread over all threads.  Four
+// barriers per term.  102,673 configurations of 6 clusters, 2 roots, FP64:
+// 508 ms when each bra state formed its own cross part and W_a summed V, 65 ms.
 template <typename T, bool DIAG>
 __global__ __launch_bounds__(RT) void k_rank1(R1Args<T> a) {
   __shared__ T sY[LMAX * RC];
   __shared__ T sX[LMAX * RC];
   __shared__ T sV[VMX];
-  __shared__ T sG0[4][NPX];     // Γ_q[:, 0, 0]
-  __shared__ T sWa[4][NPX];     // W_a
-  __shared__ T sWab[6][256];    // W_ab of the 6 cluster pairs, n_a * n_b <= 256
-  __shared__ T sU[4][NPX * RC];  // u_b[p][r]
-  __shared__ T sE;
-  __shared__ T sRed[RT];
+  __shared__ T sG[2][NPS];      // Γ_q[:, 0, 0], of this term and the last
+  __shared__ T sWa[NPS];        // W_a
+  __shared__ T sWab[WABX];      // W_ab of the cluster pairs, [p_a + n_a p_b]
+  __shared__ T sU[NPS * RC];    // u_b[p][r]
+  __shared__ T sZ[NPS * RC];    // z_a[p][r] = sum_{b != a} W_ab u_b
+  __shared__ T sW[WIJ];         // w_ij of a tile of bra states
+  __shared__ R1Ready sT[TS];
   __shared__ int sMb[FCG_MAXN], sOb[FCG_MAXN], sMk[FCG_MAXN], sOk[FCG_MAXN];
-  __shared__ int sBlk[4], sNp[4], sMbq[4], sMkq[4];
-  __shared__ int sSlotA[4];   // layout offset of each active cluster's states in F_b
-  __shared__ int sLb, sLk;
-  __shared__ int64_t sFk0;
+  __shared__ int16_t sFb[2 * FCG_MAXN], sFk[2 * FCG_MAXN];
+  __shared__ uint8_t sCl[LMAX];  // cluster of each layout slot of F_b
+  __shared__ int32_t sPk[RP], sPt0[RP], sPt1[RP], sPl[RP];
+  __shared__ int64_t sPx[RP];
 
   const int tid = threadIdx.x;
   const int64_t fb = a.fb_base + blockIdx.x;
   const int N = a.N, S = a.S, R = a.R;
-  const int16_t *Fb = a.fock + fb * 2 * N;
   if (tid < N) {
     sMb[tid] = a.meta[fb * 2 * N + tid];
     sOb[tid] = a.meta[fb * 2 * N + N + tid];
   }
-  if (tid == 0) sLb = (int)(a.foff[fb + 1] - a.foff[fb]);
-  __syncthreads();
-  const int Lb = sLb;
+  if (tid < 2 * N) sFb[tid] = a.fock[fb * 2 * N + tid];
+  const int64_t o0 = a.foff[fb];
+  const int Lb = (int)(a.foff[fb + 1] - o0);
   for (int e = tid; e < Lb * RC; e += RT) sY[e] = (T)0;
-  for (int64_t q = a.fp_ptr[fb]; q < a.fp_ptr[fb + 1]; q++) {
-    const int64_t fk = a.fp_fk[q];
-    if (DIAG && fk != fb) continue;  // only the Δ = 0 pair reaches the diagonal
-    if (!DIAG && !a.nzb[fk]) continue;  // a ket block of zeros contributes nothing
-    const int g = a.fp_g[q];
-    const int16_t *Fk = a.fock + fk * 2 * N;
-    __syncthreads();
-    if (tid < N) {
-      sMk[tid] = a.meta[fk * 2 * N + tid];
-      sOk[tid] = a.meta[fk * 2 * N + N + tid];
+  __syncthreads();
+  for (int e = tid + 1; e < Lb; e += RT) {
+    int x = 0;
+    while (x + 1 < N && sOb[x + 1] <= e) x++;
+    sCl[e] = (uint8_t)x;
+  }
+  int flip = 0;
+  const int64_t q_end = a.fp_ptr[fb + 1];
+  for (int64_t qb = a.fp_ptr[fb]; qb < q_end; qb += RP) {
+    const int np_here = (int)std::min<int64_t>(RP, q_end - qb);
+    __syncthreads();  // the last pair's readers are done
+    if (tid < np_here) {
+      const int32_t fk = a.fp_fk[qb + tid], g = a.fp_g[qb + tid];
+      // only the Δ = 0 pair reaches the diagonal; a ket block of zeros
+      // contributes nothing
+      const bool use = DIAG ? fk == fb : a.nzb[fk] != 0;
+      sPk[tid] = use ? fk : -1;
+      sPt0[tid] = a.tc_start[g];
+      sPt1[tid] = a.tc_start[g + 1];
+      sPx[tid] = a.foff[fk];
+      sPl[tid] = (int)(a.foff[fk + 1] - a.foff[fk]);
     }
-    if (tid == 0) {
-      sLk = (int)(a.foff[fk + 1] - a.foff[fk]);
-      sFk0 = a.foff[fk];
-    }
     __syncthreads();
-    const int Lk = sLk;
-    if (!DIAG)
-      for (int e = tid; e < Lk * RC; e += RT) {
-        const int i = e % Lk, r = e / Lk;
-        sX[e] = r < R ? a.x[(int64_t)r * a.n_lay + sFk0 + i] : (T)0;
+    for (int pi = 0; pi < np_here; pi++) {
+      const int64_t fk = sPk[pi];
+      if (fk < 0) continue;  // uniform
+      const int Lk = sPl[pi];
+      __syncthreads();  // the last term's readers of sX, sMk and sOk are done
+      if (tid < N) {
+        sMk[tid] = a.meta[fk * 2 * N + tid];
+        sOk[tid] = a.meta[fk * 2 * N + N + tid];
       }
-    for (int t = a.tc_start[g]; t < a.tc_start[g + 1]; t++) {
-      const R1Term Tm = a.terms[t];
-      const int nb = Tm.nbody;
-      if (nb > a.nbody) continue;
-      __syncthreads();
-      if (tid == 0) {
-        bool ok = true;
-        for (int qq = 0; qq < nb; qq++) {
-          const int c = Tm.cl[qq];
-          const int cb = Fb[2 * c] * S + Fb[2 * c + 1], ck = Fk[2 * c] * S + Fk[2 * c + 1];
-          const int SS = S * S;
-          const int blk = a.gblock[(((int64_t)c * a.n_ops + Tm.op[qq]) * SS + cb) * SS + ck];
-          sBlk[qq] = blk;
-          if (blk < 0) {
-            ok = false;
-            continue;
-          }
-          sNp[qq] = a.gb_dims[3 * blk];
-          sMbq[qq] = a.gb_dims[3 * blk + 1];
-          sMkq[qq] = a.gb_dims[3 * blk + 2];
-          sSlotA[qq] = sOb[c];
-          ok = ok && sNp[qq] <= NPX && sMbq[qq] == sMb[c] && sMkq[qq] == sMk[c];
-        }
-        if (!ok) {
-          atomicOr(a.err, 1u);
-          sBlk[0] = -1;
-        }
-      }
-      __syncthreads();
-      if (sBlk[0] < 0) continue;  // uniform; reported through err
-      // sign from the ket Fock configuration
-      T sg = (T)1;
-      {
-        int par = 0;
-        for (int qq = 0; qq < nb; qq++) {
-          if (!((Tm.odd >> qq) & 1)) continue;
-          int ne = 0;
-          for (int c2 = 0; c2 < Tm.cl[qq]; c2++) ne += Fk[2 * c2] + Fk[2 * c2 + 1];
-          par ^= ne & 1;
-        }
-        if (par) sg = (T)-1;
-      }
-      int nv = 1;
-      if (nb > 1)
-        for (int qq = 0; qq < nb; qq++) nv *= Tm.dims[qq];
-      for (int e = tid; e < nv; e += RT) sV[e] = nb > 1 ? a.ints[Tm.ioff + e] : (T)1;
-      for (int e = tid; e < 4 * NPX; e += RT) {
-        const int qq = e / NPX, p = e % NPX;
-        if (qq < nb && p < sNp[qq]) sG0[qq][p] = a.gdata[a.gb_off[sBlk[qq]] + p];
-      }
-      __syncthreads();
-      // e: fixed-order strided partial sums, then a fixed tree
-      {
-        T part = (T)0;
-        for (int v = tid; v < nv; v += RT) {
-          int p[4];
-          decode(v, nb, Tm.dims, p);
-          T f = sV[v];
-          for (int qq = 0; qq < nb; qq++) f *= sG0[qq][nb > 1 ? p[qq] : 0];
-          part += f;
-        }
-        sRed[tid] = part;
-        __syncthreads();
-        for (int s2 = RT / 2; s2 > 0; s2 >>= 1) {
-          if (tid < s2) sRed[tid] += sRed[tid + s2];
-          __syncthreads();
-        }
-        if (tid == 0) sE = sRed[0];
-      }
-      // W_a (one thread per entry) and W_ab (one thread per entry), each a
-      // fixed-order sum over the indices of the other clusters
-      int strd[4];
-      {
-        int st = 1;
-        for (int qq = 0; qq < nb; qq++) {
-          strd[qq] = st;
-          st *= nb > 1 ? Tm.dims[qq] : 1;
-        }
-      }
-      for (int e = tid; e < 4 * NPX; e += RT) {
-        const int qq = e / NPX, pq = e % NPX;
-        if (qq >= nb || pq >= sNp[qq]) continue;
-        T s = (T)0;
-        if (nb == 1) {
-          s = (T)1;
-        } else {
-          const int nrest = nv / Tm.dims[qq];
-          for (int m = 0; m < nrest; m++) {
-            int rem = m, v = pq * strd[qq];
-            T f = (T)1;
-            for (int r2 = 0; r2 < nb; r2++) {
-              if (r2 == qq) continue;
-              const int pr2 = rem % Tm.dims[r2];
-              rem /= Tm.dims[r2];
-              v += pr2 * strd[r2];
-              f *= sG0[r2][pr2];
-            }
-            s += sV[v] * f;
-          }
-        }
-        sWa[qq][pq] = s;
-      }
-      if (!DIAG && nb > 1) {
-        int pr = 0;
-        for (int qa = 0; qa < nb; qa++)
-          for (int qb = qa + 1; qb < nb; qb++, pr++) {
-            const int na = sNp[qa], nbb = sNp[qb];
-            const int nrest = nv / (Tm.dims[qa] * Tm.dims[qb]);
-            for (int e = tid; e < na * nbb; e += RT) {
-              const int pa = e % na, pb = e / na;
-              T s = (T)0;
-              for (int m = 0; m < nrest; m++) {
-                int rem = m, v = pa * strd[qa] + pb * strd[qb];
-                T f = (T)1;
-                for (int r2 = 0; r2 < nb; r2++) {
-                  if (r2 == qa || r2 == qb) continue;
-                  const int pr2 = rem % Tm.dims[r2];
-                  rem /= Tm.dims[r2];
-                  v += pr2 * strd[r2];
-                  f *= sG0[r2][pr2];
-                }
-                s += sV[v] * f;
-              }
-              sWab[pr][e] = s;
-            }
-          }
-      }
-      // u_b[p][r] = sum_{j>=1} Γ_b[p, 0, j] x_(b,j)
+      if (tid >= 64 && tid < 64 + 2 * N) sFk[tid - 64] = a.fock[fk * 2 * N + tid - 64];
       if (!DIAG)
-        for (int e = tid; e < 4 * NPX * RC; e += RT) {
-          const int qq = e / (NPX * RC), rem = e % (NPX * RC), p = rem % NPX, r = rem / NPX;
-          if (qq >= nb || p >= sNp[qq]) continue;
-          const int c = Tm.cl[qq], np = sNp[qq], mb = sMbq[qq], mk = sMkq[qq];
-          const T *G = a.gdata + a.gb_off[sBlk[qq]];
-          T s = (T)0;
-          for (int j = 1; j < mk; j++) s += G[p + (int64_t)np * (int64_t)mb * j] * sX[(sOk[c] + j - 1) + Lk * r];
-          sU[qq][p + NPX * r] = s;
+        for (int r = 0; r < R; r++)
+          for (int i = tid; i < Lk; i += RT) sX[i + Lk * r] = a.x[(int64_t)r * a.n_lay + sPx[pi] + i];
+      const int t1 = sPt1[pi];
+      for (int tb = sPt0[pi]; tb < t1; tb += TS) {
+        const int nt = min(TS, t1 - tb);
+        __syncthreads();  // sFk is there; the last batch's readers are done
+        if (tid < 4 * nt) {
+          const R1Term Tm = a.terms[tb + tid / 4];
+          R1Ready &o = sT[tid / 4];
+          const int qq = tid & 3, nb = Tm.nbody;
+          bool ok = nb <= a.nbody;
+          int np = 0;
+          if (ok && qq < nb) {
+            const int c = qq == 0 ? Tm.cl[0] : qq == 1 ? Tm.cl[1] : qq == 2 ? Tm.cl[2] : Tm.cl[3];
+            const int op = qq == 0 ? Tm.op[0] : qq == 1 ? Tm.op[1] : qq == 2 ? Tm.op[2] : Tm.op[3];
+            const int cb = sFb[2 * c] * S + sFb[2 * c + 1], ck = sFk[2 * c] * S + sFk[2 * c + 1];
+            const int SS = S * S;
+            const int blk = a.gblock[(((int64_t)c * a.n_ops + op) * SS + cb) * SS + ck];
+            if (blk < 0) {
+              ok = false;
+            } else {
+              np = a.gb_dims[3 * blk];
+              const int mb = a.gb_dims[3 * blk + 1], mk = a.gb_dims[3 * blk + 2];
+              ok = np <= NPX && mb == sMb[c] && mk == sMk[c];
+              o.goff[qq] = a.gb_off[blk];
+              o.mb[qq] = (int16_t)mb;
+              o.mk[qq] = (int16_t)mk;
+            }
+            if (!ok) atomicOr(a.err, 1u);
+            o.cl[qq] = (int16_t)c;
+          }
+          o.np[qq] = (int16_t)np;
+          // the four threads of a term agree (lanes of one wavefront)
+          const int base = (threadIdx.x & 63) & ~3;
+          bool all = true;
+          int before = 0, tot = 0;
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            all = all && __shfl((int)ok, base + k, 64);
+            const int n = __shfl(np, base + k, 64);
+            if (k < qq) before += n;
+            tot += n;
+          }
+          o.poff[qq] = (int16_t)before;
+          if (qq == 0) {
+            // sign from the ket Fock configuration
+            int par = 0, nv = 1;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+              if (k >= nb) continue;
+              if (nb > 1) nv *= Tm.dims[k];
+              if (!((Tm.odd >> k) & 1)) continue;
+              for (int c2 = 0; c2 < Tm.cl[k]; c2++) par ^= sFk[2 * c2] + sFk[2 * c2 + 1];
+            }
+            o.sgn = (par & 1) ? -1.f : 1.f;
+            o.nb = nb;
+            o.nv = nv;
+            o.ioff = Tm.ioff;
+            o.ok = all && tot <= NPS;
+          }
         }
-      __syncthreads();
-      const T e0 = sE * sg;
-      // updates: ref (threads 0..RC-1), active clusters' states, the rest
-      if (tid < RC) {
-        const int r = tid;
-        if (DIAG) {
-          if (r == 0) sY[0] += e0;
-        } else {
-          T v = sE * sX[0 + Lk * r];
-          for (int qq = 0; qq < nb; qq++)
-            for (int p = 0; p < sNp[qq]; p++) v += sWa[qq][p] * sU[qq][p + NPX * r];
-          sY[0 + Lb * r] += sg * v;
-        }
-      }
-      // active cluster qq, bra state i >= 1: thread per (qq, i)
-      for (int e = tid; e < 4 * LMAX; e += RT) {
-        const int qq = e / LMAX, i = e % LMAX;
-        if (qq >= nb || i < 1 || i >= sMbq[qq]) continue;
-        const int c = Tm.cl[qq], np = sNp[qq], mb = sMbq[qq], mk = sMkq[qq];
-        const T *G = a.gdata + a.gb_off[sBlk[qq]];
-        const int slot = sOb[c] + i - 1;
-        if (DIAG) {
-          // I = J = (c, i): W_a . Γ_a[:, i, i]
-          T d = (T)0;
-          const T *Gij = G + (int64_t)np * (i + (int64_t)mb * i);
-          for (int p = 0; p < np; p++) d += sWa[qq][p] * Gij[p];
-          sY[slot] += sg * d;
-          continue;
-        }
-        T acc[RC];
-        for (int r = 0; r < RC; r++) acc[r] = (T)0;
-        for (int j = 0; j < mk; j++) {
-          const T *Gij = G + (int64_t)np * (i + (int64_t)mb * j);
-          T w = (T)0;
-          for (int p = 0; p < np; p++) w += sWa[qq][p] * Gij[p];
-          const int xs = j == 0 ? 0 : sOk[c] + j - 1;
-          for (int r = 0; r < RC; r++) acc[r] += w * sX[xs + Lk * r];
-        }
-        // cross terms: Γ_a[:, i, 0]' W_ab u_b over the other active clusters
-        if (nb > 1) {
-          const T *Gi0 = G + (int64_t)np * i;
-          int pr = 0;
-          for (int qa = 0; qa < nb; qa++)
-            for (int qb = qa + 1; qb < nb; qb++, pr++) {
-              if (qa != qq && qb != qq) continue;
-              const int other = qa == qq ? qb : qa;
-              const int na = sNp[qa];
-              const int no = sNp[other];
-              for (int r = 0; r < RC; r++) {
-                T z = (T)0;
-                for (int pa = 0; pa < np; pa++) {
-                  T t2 = (T)0;
-                  for (int po = 0; po < no; po++) {
-                    // W_ab stored as [p_qa + n_qa * p_qb]
-                    const T w = qa == qq ? sWab[pr][pa + na * po] : sWab[pr][po + na * pa];
-                    t2 += w * sU[other][po + NPX * r];
+        __syncthreads();
+        for (int ti = 0; ti < nt; ti++) {
+          const R1Ready &t = sT[ti];
+          if (!t.ok) continue;  // uniform: dropped by nbody, or reported through err
+          const int nb = t.nb, nv = t.nv;
+          const T sg = (T)t.sgn;
+          // integrals and Γ_q[:, 0, 0]: a thread may still be in the last
+          // term's updates, which use neither this V nor this half of sG
+          flip ^= 1;
+          T *sG0 = sG[flip];
+          for (int e = tid; e < nv; e += RT) sV[e] = nb > 1 ? a.ints[t.ioff + e] : (T)1;
+          if (tid < NPS) {
+            for (int q = 0; q < nb; q++) {
+              const int p = tid - t.poff[q];
+              if (p >= 0 && p < t.np[q]) sG0[tid] = a.gdata[t.goff[q] + p];
+            }
+          }
+          __syncthreads();
+          const int d0 = nb > 1 ? t.np[0] : 1, d1 = nb > 1 ? t.np[1] : 1;
+          const int d2 = nb > 2 ? t.np[2] : 1, d3 = nb > 3 ? t.np[3] : 1;
+          // W_ab of cluster pairs (0,1) (0,2) (0,3) (1,2) (1,3) (2,3): V summed
+          // over the other clusters' g; W_ab for two clusters is V itself
+          if (nb > 1) {
+            int off = 0;
+            for (int qa = 0; qa < nb; qa++)
+              for (int qb = qa + 1; qb < nb; qb++) {
+                const int na = t.np[qa], nbb = t.np[qb];
+                const int sa = qa == 0 ? 1 : qa == 1 ? d0 : d0 * d1;
+                const int sb = qb == 1 ? d0 : qb == 2 ? d0 * d1 : d0 * d1 * d2;
+                // the other clusters (at most two), in order
+                int qc = -1, qd = -1;
+                for (int k = 0; k < nb; k++)
+                  if (k != qa && k != qb) (qc < 0 ? qc : qd) = k;
+                const int nc = qc < 0 ? 1 : t.np[qc], nd = qd < 0 ? 1 : t.np[qd];
+                const int sc = qc < 0 ? 0 : qc == 0 ? 1 : qc == 1 ? d0 : d0 * d1;
+                const int sd = qd < 0 ? 0 : qd == 1 ? d0 : qd == 2 ? d0 * d1 : d0 * d1 * d2;
+                const T *gc = sG0 + (qc < 0 ? 0 : t.poff[qc]), *gd = sG0 + (qd < 0 ? 0 : t.poff[qd]);
+                for (int e = tid; e < na * nbb; e += RT) {
+                  const T *v = sV + (e % na) * sa + (e / na) * sb;
+                  T s = (T)0;
+                  if (qc < 0) {
+                    s = v[0];
+                  } else {
+                    for (int pd = 0; pd < nd; pd++) {
+                      T s1 = (T)0;
+                      for (int pc = 0; pc < nc; pc++) s1 += v[pc * sc + pd * sd] * gc[pc];
+                      s += qd < 0 ? s1 : s1 * gd[pd];
+                    }
                   }
-                  z += Gi0[pa] * t2;
+                  sWab[off + e] = s;
                 }
-                acc[r] += z;
+                off += na * nbb;
+              }
+          }
+          // u_b[p][r] = sum_{j>=1} Γ_b[p, 0, j] x_(b,j)
+          if (!DIAG)
+            for (int e = tid; e < NPS * R; e += RT) {
+              const int pp = e % NPS, r = e / NPS;
+              for (int q = 0; q < nb; q++) {
+                const int p = pp - t.poff[q], np = t.np[q];
+                if (p < 0 || p >= np) continue;
+                const T *G = a.gdata + t.goff[q] + p;
+                const int64_t st = (int64_t)np * t.mb[q];
+                const T *x = sX + sOk[t.cl[q]] - 1 + Lk * r;
+                T s = (T)0;
+                for (int j = 1; j < t.mk[q]; j++) s += G[st * j] * x[j];
+                sU[pp + NPS * r] = s;
               }
             }
-        }
-        for (int r = 0; r < RC; r++) sY[slot + Lb * r] += sg * acc[r];
-      }
-      // clusters outside the term: (x, i) <- (x, i) with e
-      for (int e = tid; e < Lb - 1; e += RT) {
-        const int slot = e + 1;
-        // which cluster holds this slot
-        int x = 0;
-        while (x + 1 < N && sOb[x + 1] <= slot) x++;
-        bool act = false;
-        for (int qq = 0; qq < nb; qq++) act |= Tm.cl[qq] == x;
-        if (act) continue;
-        if (DIAG) {
-          sY[slot] += e0;
-        } else {
-          const int i = slot - sOb[x] + 1;  // state of cluster x (>= 1)
-          const int xs = sOk[x] + i - 1;    // the same state in the ket block
-          for (int r = 0; r < RC; r++) sY[slot + Lb * r] += e0 * sX[xs + Lk * r];
+          __syncthreads();
+          // W_a from one W_ab, and z_a from all of them
+          for (int e = tid; e < NPS * (DIAG ? 1 : 1 + R); e += RT) {
+            const int pp = e % NPS, r = e / NPS - 1;  // r = -1: W_a
+            for (int q = 0; q < nb; q++) {
+              const int p = pp - t.poff[q], np = t.np[q];
+              if (p < 0 || p >= np) continue;
+              if (nb == 1) {
+                if (r < 0) sWa[pp] = (T)1;
+                else sZ[pp + NPS * r] = (T)0;
+                continue;
+              }
+              T s = (T)0;
+              int off = 0;
+              for (int qa = 0; qa < nb; qa++)
+                for (int qb = qa + 1; qb < nb; qb++) {
+                  const int na = t.np[qa], nbb = t.np[qb];
+                  const int other = qa == q ? qb : qb == q ? qa : -1;
+                  if (other >= 0 && (r >= 0 || other == (q == 0 ? 1 : 0))) {
+                    const T *w = sWab + off + (qa == q ? p : na * p);
+                    const int st = qa == q ? na : 1, no = t.np[other];
+                    const T *f = r < 0 ? sG0 + t.poff[other] : sU + t.poff[other] + NPS * r;
+                    for (int po = 0; po < no; po++) s += w[st * po] * f[po];
+                  }
+                  off += na * nbb;
+                }
+              if (r < 0) sWa[pp] = s;
+              else sZ[pp + NPS * r] = s;
+            }
+          }
+          __syncthreads();
+          T ev = (T)0;  // e, by every thread
+          for (int p = 0; p < t.np[0]; p++) ev += sWa[p] * sG0[p];
+          // the ground configuration's row
+          if (tid < (DIAG ? 1 : R)) {
+            T v = DIAG ? ev : ev * sX[Lk * tid];
+            if (!DIAG)
+              for (int q = 0; q < nb; q++)
+                for (int p = t.poff[q]; p < t.poff[q] + t.np[q]; p++)
+                  v += sWa[p] * sU[p + NPS * tid];
+            sY[Lb * tid] += sg * v;
+          }
+          // clusters outside the term: (x, i) <- (x, i) with e
+          for (int e = RT - 1 - tid; e < Lb - 1; e += RT) {
+            const int slot = e + 1, x = sCl[slot];
+            bool act = false;
+            for (int q = 0; q < nb; q++) act |= t.cl[q] == x;
+            if (act) continue;
+            if (DIAG) {
+              sY[slot] += sg * ev;
+            } else {
+              const int xs = sOk[x] + slot - sOb[x];  // the same state in the ket block
+              for (int r = 0; r < R; r++) sY[slot + Lb * r] += sg * ev * sX[xs + Lk * r];
+            }
+          }
+          // the term's clusters, states i >= 1, in tiles of bra states whose
+          // w_ij = W_a . Γ_a[:, i, j] fit the stage
+          for (int q = 0; q < nb; q++) {
+            const int np = t.np[q], mb = t.mb[q], mk = t.mk[q], c = t.cl[q];
+            const T *G = a.gdata + t.goff[q];
+            const T *wa = sWa + t.poff[q];
+            if (DIAG) {  // I = J = (c, i): W_a . Γ_a[:, i, i]
+              for (int i = 1 + tid; i < mb; i += RT) {
+                const T *Gii = G + (int64_t)np * (i + (int64_t)mb * i);
+                T d = (T)0;
+                for (int p = 0; p < np; p++) d += wa[p] * Gii[p];
+                sY[sOb[c] + i - 1] += sg * d;
+              }
+              continue;
+            }
+            const int tile = min(mb - 1, WIJ / mk);
+            for (int i0 = 1; i0 < mb; i0 += tile) {
+              const int ni = min(tile, mb - i0);
+              if (q > 0 || i0 > 1) __syncthreads();  // the last tile's readers are done
+              for (int e = tid; e < ni * mk; e += RT) {
+                const int i = i0 + e % ni, j = e / ni;
+                const T *Gij = G + (int64_t)np * (i + (int64_t)mb * j);
+                T w = (T)0;
+                for (int p = 0; p < np; p++) w += wa[p] * Gij[p];
+                sW[e] = w;
+              }
+              __syncthreads();
+              for (int e = tid; e < ni * R; e += RT) {
+                const int k = e % ni, i = i0 + k, r = e / ni;
+                const T *x = sX + Lk * r;
+                T s = sW[k] * x[0];
+                const T *xj = x + sOk[c] - 1;
+                for (int j = 1; j < mk; j++) s += sW[k + ni * j] * xj[j];
+                if (nb > 1) {  // cross terms: Γ_a[:, i, 0]' sum_b W_ab u_b
+                  const T *Gi0 = G + (int64_t)np * i;
+                  const T *z = sZ + t.poff[q] + NPS * r;
+                  for (int p = 0; p < np; p++) s += Gi0[p] * z[p];
+                }
+                sY[sOb[c] + i - 1 + Lb * r] += sg * s;
+              }
+            }
+          }
         }
       }
     }
   }
   __syncthreads();
-  const int64_t o0 = a.foff[fb];
   if (DIAG) {
     for (int i = tid; i < Lb; i += RT) a.diag[o0 + i] = (double)sY[i];
   } else {
