@@ -107,6 +107,40 @@ constexpr int WABX = 768;   // its cluster pairs: at most 76 and 600 where every
                             // <= NPX, every pair's product <= 256 and the whole <= VMX
 constexpr int WIJ = 1024;   // staged w_ij values
 
+// the six pairs of a term's clusters, and the other two of each
+__device__ constexpr int kPa[6] = {0, 0, 0, 1, 1, 2}, kPb[6] = {1, 2, 3, 2, 3, 3};
+__device__ constexpr int kPc[6] = {2, 1, 1, 0, 0, 0}, kPd[6] = {3, 3, 2, 3, 2, 1};
+
+// a value every lane of the wavefront holds, in a scalar register
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uni64(int64_t v) {
+  const uint32_t lo = (uint32_t)uni((int)(uint32_t)v), hi = (uint32_t)uni((int)(v >> 32));
+  return (int64_t)((uint64_t)hi << 32 | lo);
+}
+
+// s + sum_k g[gs k] w[ws k], eight global loads in flight
+template <typename T>
+__device__ __forceinline__ T strided_dot(int n, const T *__restrict__ g, int64_t gs, const T *w,
+                                         int ws, T s) {
+  int k = 0;
+  for (; k + 8 <= n; k += 8) {
+    T v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = g[gs * (k + u)];
+#pragma unroll
+    for (int u = 0; u < 8; u++) s += v[u] * w[ws * (k + u)];
+  }
+  if (k < n) {  // the rest, with valid loads and zero weights past the end
+    T v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = g[gs * min(k + u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; u++)
+      if (k + u < n) s += v[u] * w[ws * (k + u)];
+  }
+  return s;
+}
+
 // a term prepared for the pair in hand
 struct R1Ready {
   int64_t goff[4], ioff;
@@ -124,7 +158,9 @@ struct R1Ready {
 // formed once per (a, p) instead of once per state of a; and the state
 // blocks' w_ij = W_a . Γ_a[:, i, j] are spread over all threads.  Four
 // barriers per term.  102,673 configurations of 6 clusters, 2 roots, FP64:
-// 508 ms when each bra state formed its own cross part and W_a summed V, 65 ms.
+// 508 ms with each bra state forming its own cross part and every W_a summing V,
+// 65 ms without, 50 ms with the shape in scalar registers and eight loads in
+// flight per dot product.
 template <typename T, bool DIAG>
 __global__ __launch_bounds__(RT) void k_rank1(R1Args<T> a) {
   __shared__ T sY[LMAX * RC];
@@ -253,119 +289,119 @@ __global__ __launch_bounds__(RT) void k_rank1(R1Args<T> a) {
         for (int ti = 0; ti < nt; ti++) {
           const R1Ready &t = sT[ti];
           if (!t.ok) continue;  // uniform: dropped by nbody, or reported through err
-          const int nb = t.nb, nv = t.nv;
+          // the term's shape in scalar registers: read from LDS where it is
+          // used, each read would cost its latency again
+          const int nb = uni(t.nb), nv = uni(t.nv);
+          int np[4], po[4], off[6];
+          const T *Gq[4];
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            np[q] = q < nb ? uni(t.np[q]) : 0;
+            po[q] = uni(t.poff[q]);
+            Gq[q] = a.gdata + (q < nb ? uni64(t.goff[q]) : 0);
+          }
+#pragma unroll
+          for (int k = 0, at = 0; k < 6; k++) {
+            off[k] = at;
+            at += np[kPa[k]] * np[kPb[k]];
+          }
           const T sg = (T)t.sgn;
           // integrals and Γ_q[:, 0, 0]: a thread may still be in the last
           // term's updates, which use neither this V nor this half of sG
           flip ^= 1;
           T *sG0 = sG[flip];
-          for (int e = tid; e < nv; e += RT) sV[e] = nb > 1 ? a.ints[t.ioff + e] : (T)1;
+          const T *ints = a.ints + uni64(t.ioff);
+          for (int e = tid; e < nv; e += RT) sV[e] = nb > 1 ? ints[e] : (T)1;
           if (tid < NPS) {
-            for (int q = 0; q < nb; q++) {
-              const int p = tid - t.poff[q];
-              if (p >= 0 && p < t.np[q]) sG0[tid] = a.gdata[t.goff[q] + p];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              const int p = tid - po[q];
+              if (p >= 0 && p < np[q]) sG0[tid] = Gq[q][p];
             }
           }
           __syncthreads();
-          const int d0 = nb > 1 ? t.np[0] : 1, d1 = nb > 1 ? t.np[1] : 1;
-          const int d2 = nb > 2 ? t.np[2] : 1, d3 = nb > 3 ? t.np[3] : 1;
-          // W_ab of cluster pairs (0,1) (0,2) (0,3) (1,2) (1,3) (2,3): V summed
-          // over the other clusters' g; W_ab for two clusters is V itself
+          // W_ab of every cluster pair: V summed over the other clusters' g;
+          // W_ab for two clusters is V itself
           if (nb > 1) {
-            int off = 0;
-            for (int qa = 0; qa < nb; qa++)
-              for (int qb = qa + 1; qb < nb; qb++) {
-                const int na = t.np[qa], nbb = t.np[qb];
-                const int sa = qa == 0 ? 1 : qa == 1 ? d0 : d0 * d1;
-                const int sb = qb == 1 ? d0 : qb == 2 ? d0 * d1 : d0 * d1 * d2;
-                // the other clusters (at most two), in order
-                int qc = -1, qd = -1;
-                for (int k = 0; k < nb; k++)
-                  if (k != qa && k != qb) (qc < 0 ? qc : qd) = k;
-                const int nc = qc < 0 ? 1 : t.np[qc], nd = qd < 0 ? 1 : t.np[qd];
-                const int sc = qc < 0 ? 0 : qc == 0 ? 1 : qc == 1 ? d0 : d0 * d1;
-                const int sd = qd < 0 ? 0 : qd == 1 ? d0 : qd == 2 ? d0 * d1 : d0 * d1 * d2;
-                const T *gc = sG0 + (qc < 0 ? 0 : t.poff[qc]), *gd = sG0 + (qd < 0 ? 0 : t.poff[qd]);
-                for (int e = tid; e < na * nbb; e += RT) {
-                  const T *v = sV + (e % na) * sa + (e / na) * sb;
-                  T s = (T)0;
-                  if (qc < 0) {
-                    s = v[0];
-                  } else {
-                    for (int pd = 0; pd < nd; pd++) {
-                      T s1 = (T)0;
-                      for (int pc = 0; pc < nc; pc++) s1 += v[pc * sc + pd * sd] * gc[pc];
-                      s += qd < 0 ? s1 : s1 * gd[pd];
-                    }
+            const int str[4] = {1, np[0], np[0] * np[1], np[0] * np[1] * np[2]};
+#pragma unroll
+            for (int k = 0; k < 6; k++) {
+              const int qa = kPa[k], qb = kPb[k];
+              if (qb >= nb) continue;
+              const int qc = kPc[k], qd = kPd[k];  // the other two, in order
+              const int na = np[qa], nc = qc < nb ? np[qc] : 1, nd = qd < nb ? np[qd] : 1;
+              for (int e = tid; e < na * np[qb]; e += RT) {
+                const T *v = sV + (e % na) * str[qa] + (e / na) * str[qb];
+                T s = (T)0;
+                if (nb == 2) {
+                  s = v[0];
+                } else {
+                  for (int pd = 0; pd < nd; pd++) {
+                    T s1 = (T)0;
+                    for (int pc = 0; pc < nc; pc++)
+                      s1 += v[pc * str[qc] + pd * str[qd]] * (qc < nb ? sG0[po[qc] + pc] : (T)1);
+                    s += qd < nb ? s1 * sG0[po[qd] + pd] : s1;
                   }
-                  sWab[off + e] = s;
                 }
-                off += na * nbb;
+                sWab[off[k] + e] = s;
               }
+            }
           }
           // u_b[p][r] = sum_{j>=1} Γ_b[p, 0, j] x_(b,j)
           if (!DIAG)
             for (int e = tid; e < NPS * R; e += RT) {
               const int pp = e % NPS, r = e / NPS;
-              for (int q = 0; q < nb; q++) {
-                const int p = pp - t.poff[q], np = t.np[q];
-                if (p < 0 || p >= np) continue;
-                const T *G = a.gdata + t.goff[q] + p;
-                const int64_t st = (int64_t)np * t.mb[q];
-                const T *x = sX + sOk[t.cl[q]] - 1 + Lk * r;
-                T s = (T)0;
-                for (int j = 1; j < t.mk[q]; j++) s += G[st * j] * x[j];
-                sU[pp + NPS * r] = s;
+#pragma unroll
+              for (int q = 0; q < 4; q++) {
+                const int p = pp - po[q];
+                if (p < 0 || p >= np[q]) continue;
+                const int mk = t.mk[q];
+                sU[pp + NPS * r] = strided_dot(mk - 1, Gq[q] + p + (int64_t)np[q] * t.mb[q],
+                                               (int64_t)np[q] * t.mb[q],
+                                               sX + sOk[t.cl[q]] + Lk * r, 1, (T)0);
               }
             }
           __syncthreads();
           // W_a from one W_ab, and z_a from all of them
           for (int e = tid; e < NPS * (DIAG ? 1 : 1 + R); e += RT) {
             const int pp = e % NPS, r = e / NPS - 1;  // r = -1: W_a
-            for (int q = 0; q < nb; q++) {
-              const int p = pp - t.poff[q], np = t.np[q];
-              if (p < 0 || p >= np) continue;
-              if (nb == 1) {
-                if (r < 0) sWa[pp] = (T)1;
-                else sZ[pp + NPS * r] = (T)0;
-                continue;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              const int p = pp - po[q];
+              if (p < 0 || p >= np[q]) continue;
+              T s = nb == 1 && r < 0 ? (T)1 : (T)0;
+#pragma unroll
+              for (int k = 0; k < 6; k++) {
+                if (kPa[k] != q && kPb[k] != q) continue;
+                const int o = kPa[k] == q ? kPb[k] : kPa[k];
+                if (o >= nb || q >= nb || (r < 0 && o != (q == 0 ? 1 : 0))) continue;
+                const T *w = sWab + off[k] + (kPa[k] == q ? p : np[o] * p);
+                const int st = kPa[k] == q ? np[q] : 1;
+                const T *f = r < 0 ? sG0 + po[o] : sU + po[o] + NPS * r;
+                for (int x = 0; x < np[o]; x++) s += w[st * x] * f[x];
               }
-              T s = (T)0;
-              int off = 0;
-              for (int qa = 0; qa < nb; qa++)
-                for (int qb = qa + 1; qb < nb; qb++) {
-                  const int na = t.np[qa], nbb = t.np[qb];
-                  const int other = qa == q ? qb : qb == q ? qa : -1;
-                  if (other >= 0 && (r >= 0 || other == (q == 0 ? 1 : 0))) {
-                    const T *w = sWab + off + (qa == q ? p : na * p);
-                    const int st = qa == q ? na : 1, no = t.np[other];
-                    const T *f = r < 0 ? sG0 + t.poff[other] : sU + t.poff[other] + NPS * r;
-                    for (int po = 0; po < no; po++) s += w[st * po] * f[po];
-                  }
-                  off += na * nbb;
-                }
               if (r < 0) sWa[pp] = s;
               else sZ[pp + NPS * r] = s;
             }
           }
           __syncthreads();
           T ev = (T)0;  // e, by every thread
-          for (int p = 0; p < t.np[0]; p++) ev += sWa[p] * sG0[p];
+          for (int p = 0; p < np[0]; p++) ev += sWa[p] * sG0[p];
           // the ground configuration's row
           if (tid < (DIAG ? 1 : R)) {
             T v = DIAG ? ev : ev * sX[Lk * tid];
-            if (!DIAG)
-              for (int q = 0; q < nb; q++)
-                for (int p = t.poff[q]; p < t.poff[q] + t.np[q]; p++)
-                  v += sWa[p] * sU[p + NPS * tid];
+            if (!DIAG) {
+              const int np_all = np[0] + np[1] + np[2] + np[3];
+              for (int p = 0; p < np_all; p++) v += sWa[p] * sU[p + NPS * tid];
+            }
             sY[Lb * tid] += sg * v;
           }
           // clusters outside the term: (x, i) <- (x, i) with e
+          const int c0 = uni(t.cl[0]), c1 = nb > 1 ? uni(t.cl[1]) : -1;
+          const int c2 = nb > 2 ? uni(t.cl[2]) : -1, c3 = nb > 3 ? uni(t.cl[3]) : -1;
           for (int e = RT - 1 - tid; e < Lb - 1; e += RT) {
             const int slot = e + 1, x = sCl[slot];
-            bool act = false;
-            for (int q = 0; q < nb; q++) act |= t.cl[q] == x;
-            if (act) continue;
+            if (x == c0 || x == c1 || x == c2 || x == c3) continue;
             if (DIAG) {
               sY[slot] += sg * ev;
             } else {
@@ -375,17 +411,16 @@ __global__ __launch_bounds__(RT) void k_rank1(R1Args<T> a) {
           }
           // the term's clusters, states i >= 1, in tiles of bra states whose
           // w_ij = W_a . Γ_a[:, i, j] fit the stage
-          for (int q = 0; q < nb; q++) {
-            const int np = t.np[q], mb = t.mb[q], mk = t.mk[q], c = t.cl[q];
-            const T *G = a.gdata + t.goff[q];
-            const T *wa = sWa + t.poff[q];
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            if (q >= nb) continue;
+            const int mb = uni(t.mb[q]), mk = uni(t.mk[q]);
+            const int ob = sOb[t.cl[q]] - 1, ok = sOk[t.cl[q]] - 1;
+            const T *wa = sWa + po[q];
             if (DIAG) {  // I = J = (c, i): W_a . Γ_a[:, i, i]
-              for (int i = 1 + tid; i < mb; i += RT) {
-                const T *Gii = G + (int64_t)np * (i + (int64_t)mb * i);
-                T d = (T)0;
-                for (int p = 0; p < np; p++) d += wa[p] * Gii[p];
-                sY[sOb[c] + i - 1] += sg * d;
-              }
+              for (int i = 1 + tid; i < mb; i += RT)
+                sY[ob + i] += sg * strided_dot(np[q], Gq[q] + (int64_t)np[q] * (i + (int64_t)mb * i),
+                                               1, wa, 1, (T)0);
               continue;
             }
             const int tile = min(mb - 1, WIJ / mk);
@@ -394,24 +429,18 @@ __global__ __launch_bounds__(RT) void k_rank1(R1Args<T> a) {
               if (q > 0 || i0 > 1) __syncthreads();  // the last tile's readers are done
               for (int e = tid; e < ni * mk; e += RT) {
                 const int i = i0 + e % ni, j = e / ni;
-                const T *Gij = G + (int64_t)np * (i + (int64_t)mb * j);
-                T w = (T)0;
-                for (int p = 0; p < np; p++) w += wa[p] * Gij[p];
-                sW[e] = w;
+                sW[e] = strided_dot(np[q], Gq[q] + (int64_t)np[q] * (i + (int64_t)mb * j), 1, wa, 1,
+                                    (T)0);
               }
               __syncthreads();
               for (int e = tid; e < ni * R; e += RT) {
                 const int k = e % ni, i = i0 + k, r = e / ni;
                 const T *x = sX + Lk * r;
                 T s = sW[k] * x[0];
-                const T *xj = x + sOk[c] - 1;
-                for (int j = 1; j < mk; j++) s += sW[k + ni * j] * xj[j];
-                if (nb > 1) {  // cross terms: Γ_a[:, i, 0]' sum_b W_ab u_b
-                  const T *Gi0 = G + (int64_t)np * i;
-                  const T *z = sZ + t.poff[q] + NPS * r;
-                  for (int p = 0; p < np; p++) s += Gi0[p] * z[p];
-                }
-                sY[sOb[c] + i - 1 + Lb * r] += sg * s;
+                for (int j = 1; j < mk; j++) s += sW[k + ni * j] * x[ok + j];
+                if (nb > 1)  // cross terms: Γ_a[:, i, 0]' sum_b W_ab u_b
+                  s = strided_dot(np[q], Gq[q] + (int64_t)np[q] * i, 1, sZ + po[q] + NPS * r, 1, s);
+                sY[ob + i + Lb * r] += sg * s;
               }
             }
           }
