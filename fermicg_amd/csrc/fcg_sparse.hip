@@ -54,7 +54,11 @@ struct SparseArgs {
   const int32_t *gb_dims;
   const double *gdata;
   int64_t fb_base;
-  int32_t *row_nnz;                  // count pass
+  // workgroups per bra Fock block, each a contiguous share of its Fock pairs
+  int parts;
+  int64_t n_row;
+  int32_t *row_nnz;                  // count pass: [parts][n_row]
+  const int32_t *part_off;           // fill pass: each part's first column in the row
   unsigned long long *stats;         // [0] triples, [1] flops, [2] missing blocks
   const int64_t *row_start;          // fill pass
   // fill pass: each TransferConfig group's terms in stage-sized chunks
@@ -415,18 +419,20 @@ __global__ __launch_bounds__(C::ST, C::WPE) void k_sparse_rows(SparseArgs a) {
   __shared__ int32_t sWave[ST / 64];
   const int tid = threadIdx.x;
   const int N = a.N;
-  const int64_t fb = a.fb_base + blockIdx.x;
+  const int64_t fb = a.fb_base + blockIdx.x / a.parts;
+  const int part = (int)(blockIdx.x % a.parts);
   const int64_t b0 = a.fstart[fb];
   const int nb = (int)(a.fstart[fb + 1] - b0);
   for (int I = tid; I < nb; I += ST) {
     pack_states(a.cfg + (b0 + I) * N, N, sPI[I]);
-    sCur[I] = 0;
+    sCur[I] = FILL ? a.part_off[part * a.n_row + b0 + I] : 0;
   }
   if (tid < 2 * N) sFb[tid] = a.fock[fb * 2 * N + tid];
   if (tid == 0) sTrip = sFlop = sMiss = 0;
   unsigned long long trip = 0, flop = 0, miss = 0;
   __syncthreads();
-  for (int64_t q = a.fp_ptr[fb]; q < a.fp_ptr[fb + 1]; q++) {
+  const int64_t qa = a.fp_ptr[fb], nq = a.fp_ptr[fb + 1] - qa;
+  for (int64_t q = qa + nq * part / a.parts; q < qa + nq * (part + 1) / a.parts; q++) {
     const int64_t fk = a.fp_fk[q];
     const int g = a.fp_g[q];
     const int64_t k0 = a.fstart[fk];
@@ -621,7 +627,7 @@ __global__ __launch_bounds__(C::ST, C::WPE) void k_sparse_rows(SparseArgs a) {
     __syncthreads();
   }
   if (!FILL)
-    for (int I = tid; I < nb; I += ST) a.row_nnz[b0 + I] = sCur[I];
+    for (int I = tid; I < nb; I += ST) a.row_nnz[part * a.n_row + b0 + I] = sCur[I];
   if (trip) atomicAdd(&sTrip, trip);
   if (flop) atomicAdd(&sFlop, flop);
   if (miss) atomicAdd(&sMiss, miss);
@@ -760,6 +766,7 @@ int upload(fcg_ctx *ctx, DBuf<T> &b, const T *src, int64_t n) {
 }
 
 constexpr int64_t FB_CHUNK = 65536;  // bra Fock blocks per launch
+constexpr int64_t JOIN_GROUPS = 4096;  // workgroups wanted of a join or fill launch
 
 uint64_t hmix64(uint64_t x) {
   x ^= x >> 33;
@@ -999,7 +1006,16 @@ int fcg_create_sparse_plan(fcg_ctx *ctx, fcg_ham *h, fcg_ops *o, fcg_space *sp, 
   if (!rc) rc = upload(ctx, d_chunk_end, chunk_end.data(), (int64_t)chunk_end.size());
   if (!rc) rc = upload(ctx, d_voff, voff.data(), (int64_t)voff.size());
   if (rc) return rc;
-  if (!d_nnz.alloc(ctx, n_row) || !d_stats.alloc(ctx, 3)) {
+  // A bra block's Fock pairs are cut into parts where there are fewer blocks
+  // than keep the chip busy to the end: one wavefront per block gives it about
+  // 3,000 at a time, and the longest block then sets the time.  More parts
+  // than that cost more than they balance, since concurrent workgroups then
+  // read different terms: whole plan build at 1, 2, 4, 8 parts 135, 116, 162,
+  // 253 ms (2,773 blocks);
+  // 31 -> 26 ms (661 blocks), 7.1 -> 4.4 ms (253 blocks) at 8.
+  int parts = 1;
+  while (parts < 8 && sp->n_fock * parts < JOIN_GROUPS) parts *= 2;
+  if (!d_nnz.alloc(ctx, parts * n_row) || !d_stats.alloc(ctx, 3)) {
     ctx->err = "device allocation failed in the sparse plan";
     return FCG_ENOMEM;
   }
@@ -1025,11 +1041,13 @@ int fcg_create_sparse_plan(fcg_ctx *ctx, fcg_ham *h, fcg_ops *o, fcg_space *sp, 
   a.gb_off = o->d_gb_off;
   a.gb_dims = o->d_gb_dims;
   a.gdata = o->d_gdata;
+  a.parts = parts;
+  a.n_row = n_row;
   a.row_nnz = d_nnz.p;
   a.stats = d_stats.p;
   for (int64_t f0 = 0; f0 < sp->n_fock; f0 += FB_CHUNK) {
     a.fb_base = f0;
-    const unsigned nblk = (unsigned)std::min<int64_t>(FB_CHUNK, sp->n_fock - f0);
+    const unsigned nblk = (unsigned)(std::min<int64_t>(FB_CHUNK, sp->n_fock - f0) * parts);
     if (small)
       hipLaunchKernelGGL((k_sparse_rows<false, SmallRows>), dim3(nblk), dim3(SmallRows::ST), 0,
                          ctx->stream, a);
@@ -1038,12 +1056,20 @@ int fcg_create_sparse_plan(fcg_ctx *ctx, fcg_ham *h, fcg_ops *o, fcg_space *sp, 
                          ctx->stream, a);
   }
   FCG_HIP(hipGetLastError(), ctx);
-  std::vector<int32_t> nnz(n_row);
+  std::vector<int32_t> part_nnz(parts * n_row);
   unsigned long long st[3];
-  FCG_HIP(hipMemcpyAsync(nnz.data(), d_nnz.p, sizeof(int32_t) * n_row, hipMemcpyDeviceToHost,
-                         ctx->stream), ctx);
+  FCG_HIP(hipMemcpyAsync(part_nnz.data(), d_nnz.p, sizeof(int32_t) * part_nnz.size(),
+                         hipMemcpyDeviceToHost, ctx->stream), ctx);
   FCG_HIP(hipMemcpyAsync(st, d_stats.p, sizeof(st), hipMemcpyDeviceToHost, ctx->stream), ctx);
   FCG_HIP(hipStreamSynchronize(ctx->stream), ctx);
+  // each part's first column in its rows, and the rows' columns
+  std::vector<int32_t> nnz(n_row, 0);
+  for (int k = 0; k < parts; k++)
+    for (int64_t b = 0; b < n_row; b++) {
+      const int32_t n = part_nnz[k * n_row + b];
+      part_nnz[k * n_row + b] = nnz[b];
+      nnz[b] += n;
+    }
   // row panels (db = 1): widths padded to whole quads
   std::vector<int64_t> col_ptr(n_row + 1, 0);
   for (int64_t b = 0; b < n_row; b++)
@@ -1108,6 +1134,11 @@ int fcg_create_sparse_plan(fcg_ctx *ctx, fcg_ham *h, fcg_ops *o, fcg_space *sp, 
       hipMemsetAsync(pl->d_diag_col, 0, sizeof(int32_t) * std::max<int64_t>(n_row, 1), s) !=
           hipSuccess)
     return fail(FCG_EDEVICE, "upload");
+  // the counts' array, read back, now holds the parts' offsets
+  if (hipMemcpyAsync(d_nnz.p, part_nnz.data(), sizeof(int32_t) * part_nnz.size(),
+                     hipMemcpyHostToDevice, s) != hipSuccess)
+    return fail(FCG_EDEVICE, "upload");
+  a.part_off = d_nnz.p;
   a.row_start = pl->d_col_ptr;
   a.K = pl->d_K64;
   a.colidx = pl->d_colidx;
@@ -1117,7 +1148,7 @@ int fcg_create_sparse_plan(fcg_ctx *ctx, fcg_ham *h, fcg_ops *o, fcg_space *sp, 
     return fail(FCG_EDEVICE, "upload");
   for (int64_t f0 = 0; f0 < sp->n_fock; f0 += FB_CHUNK) {
     a.fb_base = f0;
-    const unsigned nblk = (unsigned)std::min<int64_t>(FB_CHUNK, sp->n_fock - f0);
+    const unsigned nblk = (unsigned)(std::min<int64_t>(FB_CHUNK, sp->n_fock - f0) * parts);
     if (small)
       hipLaunchKernelGGL((k_sparse_rows<true, SmallRows>), dim3(nblk), dim3(SmallRows::ST), 0, s,
                          a);
