@@ -141,7 +141,7 @@ __device__ __forceinline__ double contract_v(const double *V, const double *cons
 
 constexpr int SV = 1536;   // staged integrals of a TransferConfig group (doubles)
 constexpr int NZMAX = 2048;  // nonzeros of one Fock pair listed for the fill (more: dense walk)
-constexpr int SVT = 64;    // staged terms per group
+constexpr int SVT = 32;    // staged terms per group
 
 // per (Fock pair, term): where each active cluster's Γ block starts, its
 // leading dimension and bra state count, and the sign; blk < 0 marks a
@@ -403,6 +403,8 @@ struct RowsCfg {
 using BigRows = RowsCfg<ST, MB, SV, SVT, NZMAX, 4>;
 using SmallRows = RowsCfg<64, 64, 512, 16, 1024, 5>;
 
+constexpr int MASKS = 32;  // terms of a pair whose masks are staged
+
 template <bool FILL, class C>
 __global__ __launch_bounds__(C::ST, C::WPE) void k_sparse_rows(SparseArgs a) {
   constexpr int ST = C::ST, MB = C::MB, SV = C::SV, SVT = C::SVT, NZMAX = C::NZ;
@@ -414,6 +416,13 @@ __global__ __launch_bounds__(C::ST, C::WPE) void k_sparse_rows(SparseArgs a) {
   __shared__ double sV[FILL ? SV : 1];
   __shared__ int32_t sVoff[FILL ? SVT : 1];
   __shared__ TermPair sTP[FILL ? SVT : 1];
+  // the chunk's terms and the pair's first terms' untouched-cluster masks, in
+  // LDS: the loops below store, so the compiler reads a term in global memory
+  // again at every use (plan build of 264,140 rows in blocks of 54: 467 -> 365
+  // ms, of 96,692 rows in blocks of 20: 156 -> 144 ms)
+  __shared__ SparseTerm sTerm[FILL ? SVT : 1];
+  __shared__ uint64_t sMask[MASKS][2];
+  __shared__ uint32_t sWork[MASKS];  // multiply-add count of the term, 0: dropped by nbody
   __shared__ uint16_t sNZ[FILL ? NZMAX : 1];  // the pair's nonzeros, (I << 8) | J
   __shared__ double sWab[FILL ? SV * 9 / 16 : 1];  // W of each factored term, 144 per 256 integrals
   __shared__ int32_t sWave[ST / 64];
@@ -440,13 +449,31 @@ __global__ __launch_bounds__(C::ST, C::WPE) void k_sparse_rows(SparseArgs a) {
     for (int J = tid; J < nk; J += ST) pack_states(a.cfg + (k0 + J) * N, N, sPJ[J]);
     if (tid < 2 * N) sFk[tid] = a.fock[fk * 2 * N + tid];
     for (int e = tid; e < nb * (MB / 64); e += ST) sBits[e / (MB / 64)][e % (MB / 64)] = 0;
-    __syncthreads();
     const int t0 = a.tc_start[g], t1 = a.tc_start[g + 1];
+    for (int t = t0 + tid; t < min(t1, t0 + MASKS); t += ST) {
+      const SparseTerm &T = a.terms[t];
+      uint32_t v = 1;
+      if (T.nbody > 1)
+        for (int k = 0; k < T.nbody; k++) v *= (uint32_t)T.dims[k];
+      sMask[t - t0][0] = T.inact[0];
+      sMask[t - t0][1] = T.inact[1];
+      sWork[t - t0] = T.nbody > a.nbody ? 0u : v;
+    }
+    __syncthreads();
     // structural nonzeros: some term passes check_term
     for (int e = tid; e < nb * nk; e += ST) {
       const int I = e / nk, J = e % nk;
       bool nz = false;
-      for (int t = t0; t < t1; t++) {
+      const uint64_t x0 = sPI[I][0] ^ sPJ[J][0], x1 = sPI[I][1] ^ sPJ[J][1];
+      for (int t = 0; t < min(t1 - t0, MASKS); t++) {
+        const uint32_t v = sWork[t];
+        if (v == 0 || (x0 & sMask[t][0]) || (x1 & sMask[t][1])) continue;
+        nz = true;
+        if (FILL) break;
+        trip++;
+        flop += 2 * (uint64_t)v;
+      }
+      for (int t = t0 + MASKS; t < t1; t++) {
         const SparseTerm &T = a.terms[t];
         if (T.nbody > a.nbody) continue;
         if (((sPI[I][0] ^ sPJ[J][0]) & T.inact[0]) | ((sPI[I][1] ^ sPJ[J][1]) & T.inact[1]))
@@ -507,13 +534,14 @@ __global__ __launch_bounds__(C::ST, C::WPE) void k_sparse_rows(SparseArgs a) {
       for (int c0 = t0, first = 1, kc = a.grp_chunk[g]; c0 < t1; first = 0, kc++) {
         const int c1 = a.chunk_end[kc];
         for (int t = c0 + tid; t < c1; t += ST) {
+          sTerm[t - c0] = a.terms[t];
           sVoff[t - c0] = a.voff[t];
           term_pair(a, a.terms[t], sFb, sFk, &sTP[t - c0]);
         }
         __syncthreads();
         for (int t = c0; t < c1; t++) {
           const int off = sVoff[t - c0];
-          const SparseTerm &T = a.terms[t];
+          const SparseTerm &T = sTerm[t - c0];
           if (off < 0 || T.nbody == 1) continue;  // skipped, or integrals left in global memory
           int sz = 1;
           for (int k = 0; k < T.nbody; k++) sz *= T.dims[k];
@@ -524,7 +552,7 @@ __global__ __launch_bounds__(C::ST, C::WPE) void k_sparse_rows(SparseArgs a) {
         if (fact) {
           for (int t = c0; t < c1; t++) {
             const int off = sVoff[t - c0];
-            const SparseTerm &T = a.terms[t];
+            const SparseTerm &T = sTerm[t - c0];
             if (off < 0 || T.nbody < 3) continue;
             const int id = shape_id(T);
             const TermPair &tp = sTP[t - c0];
@@ -548,7 +576,7 @@ __global__ __launch_bounds__(C::ST, C::WPE) void k_sparse_rows(SparseArgs a) {
           double v = 0.0;
           bool ms = false;
           for (int t = c0; t < c1; t++) {
-            const SparseTerm &T = a.terms[t];
+            const SparseTerm &T = sTerm[t - c0];
             const int off = sVoff[t - c0];
             if (off == -1) continue;
             if (((sPI[I][0] ^ sPJ[J][0]) & T.inact[0]) | ((sPI[I][1] ^ sPJ[J][1]) & T.inact[1]))
