@@ -1,6 +1,6 @@
 """Davidson where its tall-skinny products have edges: spaces around a stage
-of rows (128) and the rounds of stages, root counts below, at and above an
-output tile (8 columns), and subspaces above the GPU eigensolver's limit.
+of rows (128) and a round of four stages, and root counts below and above an
+output tile (8 columns).
 
 Reference: the eigenvalues and residuals of the dense H of the same space
 (build_full_H, symmetrised).  Bars: the solver stops at a residual norm of
