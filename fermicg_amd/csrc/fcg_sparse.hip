@@ -391,15 +391,15 @@ __device__ __forceinline__ double contract_factored(int nbody, const int32_t *d,
 // chunk, and the longest listed nonzero list per Fock pair.  Spaces whose
 // Fock blocks hold at most 64 configurations take one wavefront per bra
 // block with small stages: a Fock pair has ~90 nonzeros, which leave most of
-// a 256-thread workgroup idle, and the smaller LDS footprint (10 KB against
-// 38 KB) fits four times as many workgroups per CU.
+// a 256-thread workgroup idle, and the smaller LDS footprint (15 KB against
+// 47 KB) fits three times as many workgroups per CU.
 template <int ST_, int MB_, int SV_, int SVT_, int NZ_, int WPE_>
 struct RowsCfg {
   static constexpr int ST = ST_, MB = MB_, SV = SV_, SVT = SVT_, NZ = NZ_, WPE = WPE_;
 };
-// WPE: the waves per SIMD asked of the register allocator (the small
-// variant then fits 128 VGPRs without scratch: four waves per SIMD, which its
-// 10 KB of LDS also allows)
+// WPE: the launch bound's second figure; the fill then takes 154 (small) and
+// 162 registers without scratch: three waves per SIMD, about what the LDS of
+// either shape allows
 using BigRows = RowsCfg<ST, MB, SV, SVT, NZMAX, 4>;
 using SmallRows = RowsCfg<64, 64, 512, 16, 1024, 5>;
 
