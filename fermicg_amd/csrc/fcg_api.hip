@@ -559,8 +559,8 @@ int fcg_create_plan(fcg_ctx *ctx, fcg_ham *h, fcg_ops *o, fcg_space *sp, fcg_spa
     PTRY(dev_upload(ctx, &pl->d_order, hp.order.data(), (int64_t)hp.order.size()));
     pl->n_multi = hp.n_multi;
     pl->n_single_slots = hp.n_single_slots;
-    pl->n_split = hp.n_split;
-    pl->split_parts = fcg_split_parts(hp.n_split);
+    pl->mean_panel = hp.mean_panel;
+    pl->split_parts = fcg_split_parts(hp.n_multi);
     pl->n_single = hp.n_single;
     PTRY(dev_upload(ctx, &pl->d_colidx, hp.colidx.data(), pl->n_cols));
   }

@@ -38,21 +38,33 @@ constexpr int FCG_MAX_R = 16;         // roots per sigma launch
 constexpr int FCG_N_PREC = 5;  // FCG_FP64 .. FCG_FP32_BF16C
 constexpr int FCG_QUAD = 4;           // panel columns per stored column quad
 constexpr int FCG_CSR_WPB = 4;        // one-row boxes: wavefronts (rows) per workgroup
-// Plans with fewer multi-row boxes than this share each panel of at least
-// FCG_SHARE_MIN elements between the wavefronts of a workgroup
-// (k_apply_stream); with more, one wavefront per box (k_apply) already fills
-// the chip and wastes less on short panels.  Measured, shared against not:
-// 73 boxes FP64 58 / 110 us; 2,380 boxes FP32 288 / 541 us; 9,408 boxes FP64
-// 1.95 / 2.83 ms; 28,784 boxes FP64 10.1 / 10.2 ms but FP32 6.5 / 5.5 ms.
-// Sharing only the largest panels leaves two launches, each with its own
-// tail: 28,784 boxes FP32 5.8-6.4 ms.
-constexpr int64_t FCG_SHARE_BOXES = 16384, FCG_SHARE_MIN = 8192;
+// Multi-row boxes have two kernels with the same sums: k_apply_stream shares
+// a panel's loads between the wavefronts of a workgroup, k_apply gives a box
+// one wavefront.  With this many boxes one wavefront per box already fills
+// the chip (28,784 boxes, shared against not: FP64 10.1 / 10.2 ms, FP32
+// 6.5 / 5.5 ms).  With fewer, which is faster depends on the panels' sizes,
+// the roots and the precision, so both are among the timed variants.  All of
+// a plan's boxes take the same one: the two kernels one after the other have
+// a tail each (2,022 boxes of 4,553 elements, FP64, 1 root: 60 us shared from
+// 8,192 elements up, 46 none shared, 61 all; 2,258 of 17,512: 116, 118, 104).
+constexpr int64_t FCG_SHARE_BOXES = 16384;
+// Above the timed root count a rule decides, by the bytes of c
+// gathered per column: k_apply keeps the roots' sums of a lane in one
+// wavefront, k_apply_stream divides them over four.  mean: elements per box.
+// Shared / not, us: FP64 8 roots 161 / 244 (2,022 boxes, mean 4,553), 589 /
+// 1001 (8,055, 8,891), 91 / 91 (363, 3,367); FP64 5 roots 381 / 503 (8,055,
+// 8,891), 94 / 118 (2,022, 4,553); FP64 6 roots 68 / 63 (363, 3,367); FP32 10
+// roots 358 / 408 (8,055, 8,891); FP32 8 roots 103 / 119 (2,022, 4,553),
+// 392 / 341 (8,055, 8,891), 514 / 511 (8,657, 19,162), 801 / 947 (8,963, 37,601).
+inline bool fcg_share_untimed(int64_t n_boxes, int64_t mean, int c_bytes) {
+  return c_bytes >= 40 ? mean >= 4096 : mean >= (n_boxes < 4096 ? 4096 : 32768);
+}
 // Row groups (workgroups) per shared panel: enough for two workgroups per CU,
 // at most eight of a 64-row panel (a group's rows then read 128-byte runs of
 // FP32).  73 panels of 64 rows, FP64: 69 us in four groups, 58 in eight.
-inline int fcg_split_parts(int64_t n_split) {
+inline int fcg_split_parts(int64_t n_boxes) {
   int p = 1;
-  while (p < 8 && n_split > 0 && n_split * p < 512) p *= 2;
+  while (p < 8 && n_boxes > 0 && n_boxes * p < 512) p *= 2;
   return p;
 }
 // Plans with fewer one-row boxes than this share each between this many
@@ -196,8 +208,8 @@ struct fcg_plan {
   // that each XCD's workgroups take a contiguous run of rows
   int32_t *d_order = nullptr;
   int64_t n_multi = 0, n_single_slots = 0;
-  int64_t n_split = 0;   // the first boxes of the order, applied by k_apply_stream
-  int split_parts = 1;   // ... in this many row groups each (fcg_split_parts)
+  int64_t mean_panel = 0;  // elements per box of several rows
+  int split_parts = 1;     // k_apply_stream's row groups per box (fcg_split_parts)
   int64_t n_single = 0;  // one-row boxes
   int32_t *d_colidx = nullptr;    // [n_cols] column -> variable index
   int64_t n_cols = 0;
@@ -266,7 +278,7 @@ struct HostPlan {
   RawVec<int64_t> pair_t0, pair_koff;
   std::vector<int64_t> row_ptr, diag_koff, row_koff, col_ptr;
   std::vector<int32_t> diag_col, order;
-  int64_t n_multi = 0, n_single_slots = 0, n_split = 0, n_single = 0;
+  int64_t n_multi = 0, n_single_slots = 0, mean_panel = 0, n_single = 0;
   RawVec<TaskDev> tasks;
   // pair indices for the block build: pairs within the tiny class's limits
   // first (n_tiny of them; plans that store their blocks only), then those
@@ -281,7 +293,7 @@ struct HostPlan {
 // apply schedule of a plan (see fcg_plan::d_order)
 void fcg_apply_order(const std::vector<int64_t> &var_off, const std::vector<int64_t> &col_ptr,
                      std::vector<int32_t> *order, int64_t *n_multi, int64_t *n_single_slots,
-                     int64_t *n_split, int64_t *n_single);
+                     int64_t *mean_panel, int64_t *n_single);
 // layout = false: pairs, tasks and LDS classes only (a plan whose blocks are
 // used once during the build); pair_col, pair_koff, the row panels, colidx,
 // the apply order and the diagonal tables are left empty

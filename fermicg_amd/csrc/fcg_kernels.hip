@@ -425,7 +425,9 @@ __device__ __forceinline__ float kval(uint16_t u) {  // bf16
 // the result does not depend on the choice.
 //   multi-row boxes (k_apply): wavefronts per workgroup, quads in flight;
 //     32-bit blocks load branch-free from a clamped quad, 64-bit ones
-//     predicated (measured faster each way);
+//     predicated (measured faster each way).  Plans of fewer than
+//     FCG_SHARE_BOXES of them choose between k_apply_stream and k_apply
+//     (launch_multi_v);
 //   one-row boxes (k_apply_rows): quads in flight.
 struct MultiVariant { int wpb, unroll; bool nt; };
 constexpr MultiVariant kMulti[] = {{4, 16, false}, {1, 16, false}, {4, 8, false},
@@ -713,7 +715,7 @@ __global__ __launch_bounds__(64 * WPB) void k_apply(int64_t n_box,
   }
 }
 
-// The larger panels of a plan (fcg_plan::n_split): one workgroup per bra box
+// Multi-row boxes with their panels shared: one workgroup per bra box
 // (or per group of its rows, `parts` groups) streams the panel through LDS.
 // The sums are k_apply's, term by term: row i's slice s takes the quads j of
 // each CG-quad chunk with (j mod CG) mod sl == s in order, and the slices are
@@ -1166,23 +1168,39 @@ hipError_t fcg_launch_convert(const fcg_plan *pl, hipStream_t s) {
   return hipGetLastError();
 }
 
+// On a plan of fewer than FCG_SHARE_BOXES multi-row boxes the variants are
+// k_apply_stream with 16 KB stages (the default), the same with non-temporal
+// loads (3), with 8 KB stages (4), and k_apply with 8 (2) and 16 quads in
+// flight (the latter non-temporal for blocks of 32 and 16 bits): what won
+// most often of each kernel's forms over thirteen Tucker spaces.  Above TUNED_MAX_R only the default is compiled, and the rule
+// fcg_share_untimed decides between the kernels.
 template <typename TK, typename TA, typename TC, int R, int V>
 void launch_multi_v(const fcg_plan *pl, const TK *K, const TC *c, double *sigma, hipStream_t s) {
-  constexpr int W = kMulti[V].wpb, U = kMulti[V].unroll;
-  constexpr bool NT = kMulti[V].nt;
-  const int64_t ns = pl->n_split, n1 = pl->n_multi - ns;
-  if (ns > 0) {
-    constexpr int SB = (U >= 16 ? 16384 : 8192) / (sizeof(TK) == 2 ? 2 : 1);
-    hipLaunchKernelGGL((k_apply_stream<TK, TA, TC, R, SB, NT>),
-                       dim3((unsigned)(ns * pl->split_parts)), dim3(256), 0, s, pl->split_parts,
-                       pl->d_order, pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr, pl->d_colidx, K,
-                       c, pl->sp->nvar, sigma);
-  }
-  if (n1 > 0)
-    hipLaunchKernelGGL((k_apply<TK, TA, TC, R, W, U, apply_clamp<TK>(), NT>),
-                       dim3((unsigned)((n1 + W - 1) / W)), dim3(64 * W), 0, s, n1,
-                       pl->d_order + ns, pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr,
+  constexpr bool DEF = V == default_multi<TK>();
+  auto stream = [&] {
+    constexpr int SB = (V == 4 ? 8192 : 16384) / (sizeof(TK) == 2 ? 2 : 1);
+    hipLaunchKernelGGL((k_apply_stream<TK, TA, TC, R, SB, V == 3>),
+                       dim3((unsigned)(pl->n_multi * pl->split_parts)), dim3(256), 0, s,
+                       pl->split_parts, pl->d_order, pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr,
                        pl->d_colidx, K, c, pl->sp->nvar, sigma);
+  };
+  auto boxes = [&](auto form) {
+    constexpr MultiVariant F = kMulti[decltype(form)::value];
+    hipLaunchKernelGGL((k_apply<TK, TA, TC, R, F.wpb, F.unroll, apply_clamp<TK>(), F.nt>),
+                       dim3((unsigned)((pl->n_multi + F.wpb - 1) / F.wpb)), dim3(64 * F.wpb), 0, s,
+                       pl->n_multi, pl->d_order, pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr,
+                       pl->d_colidx, K, c, pl->sp->nvar, sigma);
+  };
+  if (pl->n_multi >= FCG_SHARE_BOXES) {
+    boxes(std::integral_constant<int, V>{});
+  } else if constexpr (R > TUNED_MAX_R) {
+    if (fcg_share_untimed(pl->n_multi, pl->mean_panel, R * (int)sizeof(TC))) stream();
+    else boxes(std::integral_constant<int, V>{});
+  } else if constexpr (DEF || V >= 3) {
+    stream();
+  } else {
+    boxes(std::integral_constant<int, V == 2 ? 2 : sizeof(TK) == 8 ? 1 : 4>{});
+  }
 }
 
 template <typename TK, typename TA, typename TC, int R, int V>

@@ -649,7 +649,7 @@ int fcg_build_host_plan(const fcg_ham *h, const fcg_ops *o, const fcg_space *bra
     for (; at < out->col_ptr[b + 1]; at++) out->colidx[at] = 0;  // padding columns
   }
   fcg_apply_order(bra->var_off, out->col_ptr, &out->order, &out->n_multi, &out->n_single_slots,
-                  &out->n_split, &out->n_single);
+                  &out->mean_panel, &out->n_single);
   out->n_kel = koff;
   return FCG_OK;
 }
@@ -866,7 +866,7 @@ int fcg_fock_pairs(const fcg_ham *h, const fcg_space *bra, const fcg_space *ket,
 // (g mod 8) * G + g / 8 and each XCD's L2 sees one contiguous run of rows.
 void fcg_apply_order(const std::vector<int64_t> &var_off, const std::vector<int64_t> &col_ptr,
                      std::vector<int32_t> *order, int64_t *n_multi, int64_t *n_single_slots,
-                     int64_t *n_split, int64_t *n_single) {
+                     int64_t *mean_panel, int64_t *n_single) {
   const int64_t n_box = (int64_t)var_off.size() - 1;
   std::vector<int32_t> multi, single;
   for (int64_t b = 0; b < n_box; b++)
@@ -876,9 +876,9 @@ void fcg_apply_order(const std::vector<int64_t> &var_off, const std::vector<int6
   };
   std::stable_sort(multi.begin(), multi.end(),
                    [&](int32_t a, int32_t b) { return size(a) > size(b); });
-  *n_split = 0;
-  if ((int64_t)multi.size() < FCG_SHARE_BOXES)
-    while (*n_split < (int64_t)multi.size() && size(multi[*n_split]) >= FCG_SHARE_MIN) ++*n_split;
+  *mean_panel = 0;
+  for (int32_t b : multi) *mean_panel += size(b);
+  if (!multi.empty()) *mean_panel /= (int64_t)multi.size();
   const int64_t ns = (int64_t)single.size();
   const int64_t nw = (ns + FCG_CSR_WPB - 1) / FCG_CSR_WPB;
   const int64_t g8 = (nw + FCG_XCDS - 1) / FCG_XCDS;

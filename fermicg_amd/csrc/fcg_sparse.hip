@@ -1124,7 +1124,7 @@ int fcg_create_sparse_plan(fcg_ctx *ctx, fcg_ham *h, fcg_ops *o, fcg_space *sp, 
   std::vector<int64_t> var_off(n_row + 1);
   std::iota(var_off.begin(), var_off.end(), 0);
   fcg_apply_order(var_off, col_ptr, &order, &pl->n_multi, &pl->n_single_slots,
-                  &pl->n_split, &pl->n_single);
+                  &pl->mean_panel, &pl->n_single);
   auto fail = [&](int code, const char *what) {
     if (code == FCG_EDEVICE || code == FCG_ENOMEM) ctx->err = std::string("sparse plan: ") + what;
     fcg_plan_destroy(pl);

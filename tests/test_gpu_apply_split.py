@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+from fermicg_amd import _lib
 from fermicg_amd.bst import bst_pq_state, cache_hamiltonian
 from fermicg_amd.marshal import flatten_ham, flatten_ops
 from fermicg_amd.state import TPSCIstate
@@ -61,6 +62,31 @@ def test_tucker_boxes(eng, clusters, M, rank, R):
     plan = cache_hamiltonian(st, st, p.cluster_ops, p.clustered_ham, precisions=tuple(TOL),
                              engine=eng)
     _check(plan, ref, st.coeffs, (clusters, M, rank, R))
+    eng.drop_plans()
+
+
+@pytest.mark.parametrize("clusters,M,rank,R", [(3, 5, 2, 1), (3, 8, 4, 2), (3, 12, 6, 4), (2, 3, 1, 3),
+                                               (3, 8, 4, 6), (3, 12, 6, 5), (3, 9, 7, 12)])
+def test_shared_and_unshared_panels(eng, clusters, M, rank, R):
+    """Panels of a few to 60,000 elements through every form of the multi-row
+    apply, the ones that share a panel and the ones that do not: the same
+    bits (up to four roots; above, the one the rule takes), and the oracle's
+    sigma."""
+    p = build_problem(4 * clusters, clusters, M, 8 * clusters, seed=M, max_transfer=2)
+    st = bst_pq_state(p.bases, p.focks, p.ref_fock, max_rank=rank, R=R, seed=rank)
+    ref = BstOracle(flatten_ops(p.cluster_ops, cluster_sizes_of(p.cluster_ops)),
+                    flatten_ham(p.clustered_ham), st).sigma_rows(st.coeffs,
+                                                                np.arange(len(st.blocks)))[0]
+    plan = cache_hamiltonian(st, st, p.cluster_ops, p.clustered_ham, precisions=tuple(TOL),
+                             engine=eng)
+    nm, nr, max_r = _lib.apply_variant_counts()
+    _check(plan, ref, st.coeffs, (clusters, M, rank, R))
+    for prec in TOL if R <= max_r else ():
+        got = []
+        for v in range(nm):
+            plan.set_apply_variant(prec, R, v, 0)
+            got.append(plan.sigma(st.coeffs, prec))
+        assert all(np.array_equal(g, got[0]) for g in got), prec
     eng.drop_plans()
 
 
