@@ -67,12 +67,14 @@ inline int fcg_split_parts(int64_t n_boxes) {
   while (p < 8 && n_boxes > 0 && n_boxes * p < 512) p *= 2;
   return p;
 }
-// Plans with fewer one-row boxes than this share each between this many
-// wavefronts (FP64 sums only: FP32 ones keep the order, and so the rounding,
-// of a wavefront per row).  661 rows of 10,000 columns: 128 us with a
-// wavefront each, 20 shared.
+// FP64 plans with fewer one-row boxes than this share a row's loads between
+// the wavefronts of a workgroup (k_apply_row_stream: the sums of a wavefront
+// per row, bit for bit).  1,168 rows of 10,922 columns, 2 roots: 128 us with
+// a wavefront each, 71 shared.  A whole sigma, shared against not, 2 / 16 roots:
+// 236 rows of 282 columns 27 / 103 and 28 / 114 us; 1,613 of 5,426 648 /
+// 2,457 and 676 / 2,856; 2,449 of 842 27 / 81 and 23 / 82; 10,809 of 1,824
+// 86 / 528 and 63 / 442.
 constexpr int64_t FCG_SHARED_ROWS = 2048;
-constexpr int FCG_ROW_WAVES = 8;
 constexpr int FCG_XCDS = 8;           // MI355X accelerator complex dies (workgroups round-robin)
 
 // Row panel storage.  The Hamiltonian blocks of one bra box (db rows) sit

@@ -935,20 +935,16 @@ __global__ __launch_bounds__(256) void k_apply_stream(
 // instruction (1.45x over quad-per-lane gathers on the 2e6-configuration
 // rank-1 space).  Rows come from `order` (XCD-grouped slots, -1 = empty);
 // the 64 lane sums are combined by a fixed butterfly.
-// WPR = 1: a workgroup's wavefronts take a row each.  WPR > 1: they
-// share one row, a contiguous part each, summed in order -- for plans with
-// fewer rows than the chip holds wavefronts (FCG_SHARED_ROWS).
-template <typename TK, typename TA, typename TC, int R, int U, bool NT, int WPR>
-__global__ __launch_bounds__(64 * (WPR > 1 ? WPR : FCG_CSR_WPB)) void k_apply_rows(
+template <typename TK, typename TA, typename TC, int R, int U, bool NT>
+__global__ __launch_bounds__(64 * FCG_CSR_WPB) void k_apply_rows(
     int64_t n_slots, const int32_t *__restrict__ order, const int64_t *__restrict__ var,
     const int64_t *__restrict__ row_koff, const int64_t *__restrict__ col_ptr,
     const int32_t *__restrict__ colidx, const TK *__restrict__ K, const TC *__restrict__ c,
     int64_t nvar_s, double *__restrict__ sigma) {
-  __shared__ TA sPart[WPR][R];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t w = WPR > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * FCG_CSR_WPB + wave;
+  const int64_t w = (int64_t)blockIdx.x * FCG_CSR_WPB + wave;
   const int32_t b = w < n_slots ? order[w] : -1;
-  if (b < 0) return;  // uniform per wave (and per workgroup when it shares a row)
+  if (b < 0) return;  // uniform per wave
   const int64_t c0 = col_ptr[b];
   const int ngrp = (int)((col_ptr[b + 1] - c0) / FCG_QUAD);
   const TK *Kr = K + row_koff[b];
@@ -956,16 +952,11 @@ __global__ __launch_bounds__(64 * (WPR > 1 ? WPR : FCG_CSR_WPB)) void k_apply_ro
   TA acc[R];
 #pragma unroll
   for (int r = 0; r < R; r++) acc[r] = (TA)0;
-  int first = 0, ncol = FCG_QUAD * ngrp;
-  if (WPR > 1) {
-    const int per = (ncol + 64 * WPR - 1) / (64 * WPR) * 64;
-    first = per * wave;
-    ncol = min(ncol, first + per);
-  }
+  const int ncol = FCG_QUAD * ngrp;
   const TK *Kl = Kr + lane;
   const int32_t *cl = ci + lane;
   constexpr int NE = 4 * U;  // columns in flight per lane
-  for (int s0 = first; s0 < ncol; s0 += 64 * NE) {
+  for (int s0 = 0; s0 < ncol; s0 += 64 * NE) {
     TK kv[NE];
     int idx[NE];
 #pragma unroll
@@ -995,20 +986,97 @@ __global__ __launch_bounds__(64 * (WPR > 1 ? WPR : FCG_CSR_WPB)) void k_apply_ro
     for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
     acc[r] = v;
   }
-  if (WPR > 1) {
-    if (lane == 0) {
-#pragma unroll
-      for (int r = 0; r < R; r++) sPart[wave][r] = acc[r];
-    }
-    __syncthreads();
-    if (threadIdx.x < R) {
-      TA v = (TA)0;
-      for (int k = 0; k < WPR; k++) v += sPart[k][threadIdx.x];
-      sigma[(int64_t)threadIdx.x * nvar_s + var[b]] = (double)v;
-    }
-  } else if (lane == 0) {
+  if (lane == 0) {
 #pragma unroll
     for (int r = 0; r < R; r++) sigma[(int64_t)r * nvar_s + var[b]] = (double)acc[r];
+  }
+}
+
+// The same rows and sums where there are fewer rows than the chip holds
+// wavefronts: one workgroup per row.  All eight wavefronts load tiles of
+// T columns, D tiles ahead of the one in use, and pass them through LDS;
+// wavefront w then runs root w's 64 chains (lane l: columns l, l+64, ...)
+// and w + 8's.  Bound by the round trips index -> c, which the tiles in
+// flight divide; the chains are a few steps per tile.
+template <typename TK, typename TA, typename TC, int R, bool NT>
+__global__ __launch_bounds__(512) void k_apply_row_stream(
+    const int32_t *__restrict__ order, const int64_t *__restrict__ var,
+    const int64_t *__restrict__ row_koff, const int64_t *__restrict__ col_ptr,
+    const int32_t *__restrict__ colidx, const TK *__restrict__ K, const TC *__restrict__ c,
+    int64_t nvar_s, double *__restrict__ sigma) {
+  constexpr int T = R <= 8 ? 512 : 256;  // at most 37 KB of LDS
+  constexpr int D = R <= 4 ? 4 : 2;
+  constexpr int NR = (R + 7) / 8;  // roots per wavefront
+  __shared__ TK sK[T];
+  __shared__ TC sC[R][T];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int32_t b = order[blockIdx.x];
+  if (b < 0) return;  // uniform
+  const int64_t c0 = col_ptr[b];
+  const int ncol = (int)(col_ptr[b + 1] - c0);
+  const TK *Kr = K + row_koff[b];
+  const int32_t *ci = colidx + c0;
+  const int nt = (ncol + T - 1) / T;
+  const int p = tid < T ? tid : 0;  // this thread's column of a tile
+  TK kv[D];
+  TC cv[D][R];
+  int idx[D];
+  // columns past the row's end are loaded from its last one and stand for
+  // zero elements of column 0, as in k_apply_rows
+  auto load_idx = [&](int t, int d) {
+    const int j = t * T + p;
+    const int i = ld_stream<NT>(ci + min(j, ncol - 1));
+    idx[d] = j < ncol ? i : 0;
+  };
+  auto load = [&](int t, int d) {
+    const int j = t * T + p;
+    const TK k = ld_stream<NT>(Kr + min(j, ncol - 1));
+    kv[d] = j < ncol ? k : (TK)0;
+    load_row<TC, R>(c + (int64_t)idx[d] * R, cv[d]);
+  };
+  TA acc[NR];
+#pragma unroll
+  for (int m = 0; m < NR; m++) acc[m] = (TA)0;
+  if (nt > 0) {
+#pragma unroll
+    for (int d = 0; d < D; d++) load_idx(d, d);
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      load(d, d);
+      load_idx(d + D, d);
+    }
+    for (int t0 = 0; t0 < nt; t0 += D) {
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        const int t = t0 + d;
+        if (t >= nt) break;  // uniform
+        __syncthreads();  // the last tile's readers are done
+        if (tid < T) {
+          sK[tid] = kv[d];
+#pragma unroll
+          for (int r = 0; r < R; r++) sC[r][tid] = cv[d][r];
+        }
+        load(t + D, d);
+        load_idx(t + 2 * D, d);
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < NR; m++) {
+          const int r = wave + 8 * m;
+          if (r >= R) continue;
+#pragma unroll
+          for (int e = 0; e < T / 64; e++)
+            acc[m] += kval(sK[64 * e + lane]) * (TA)sC[r][64 * e + lane];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < NR; m++) {
+    const int r = wave + 8 * m;
+    TA v = acc[m];
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) v += __shfl_xor(v, s, 64);
+    if (lane == 0 && r < R) sigma[(int64_t)r * nvar_s + var[b]] = (double)v;
   }
 }
 
@@ -1205,22 +1273,19 @@ void launch_multi_v(const fcg_plan *pl, const TK *K, const TC *c, double *sigma,
 
 template <typename TK, typename TA, typename TC, int R, int V>
 void launch_rows_v(const fcg_plan *pl, const TK *K, const TC *c, double *sigma, hipStream_t s) {
-  auto launch = [&](auto wpr) {
-    constexpr int W = decltype(wpr)::value;
-    const int64_t n = pl->n_single_slots;
-    hipLaunchKernelGGL((k_apply_rows<TK, TA, TC, R, kRows[V].unroll, kRows[V].nt, W>),
-                       dim3((unsigned)(W > 1 ? n : n / FCG_CSR_WPB)),
-                       dim3(64 * (W > 1 ? W : FCG_CSR_WPB)), 0, s, n, pl->d_order + pl->n_multi,
-                       pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr, pl->d_colidx, K, c,
-                       pl->sp->nvar, sigma);
-  };
+  const int64_t n = pl->n_single_slots;
   if constexpr (sizeof(TA) == 8) {
     if (pl->n_single < FCG_SHARED_ROWS) {
-      launch(std::integral_constant<int, FCG_ROW_WAVES>{});
+      hipLaunchKernelGGL((k_apply_row_stream<TK, TA, TC, R, kRows[V].nt>), dim3((unsigned)n),
+                         dim3(512), 0, s, pl->d_order + pl->n_multi, pl->sp->d_var, pl->d_row_koff,
+                         pl->d_col_ptr, pl->d_colidx, K, c, pl->sp->nvar, sigma);
       return;
     }
   }
-  launch(std::integral_constant<int, 1>{});
+  hipLaunchKernelGGL((k_apply_rows<TK, TA, TC, R, kRows[V].unroll, kRows[V].nt>),
+                     dim3((unsigned)(n / FCG_CSR_WPB)), dim3(64 * FCG_CSR_WPB), 0, s, n,
+                     pl->d_order + pl->n_multi, pl->sp->d_var, pl->d_row_koff, pl->d_col_ptr,
+                     pl->d_colidx, K, c, pl->sp->nvar, sigma);
 }
 
 // parts: bit 0 multi-row boxes, bit 1 one-row boxes

@@ -16,7 +16,7 @@ from fermicg_amd.bst import bst_pq_state, cache_hamiltonian
 from fermicg_amd.marshal import flatten_ham, flatten_ops
 from fermicg_amd.state import TPSCIstate
 from fermicg_amd.tpsci import Engine, cluster_sizes_of
-from fermicg_amd.workloads import build_problem
+from fermicg_amd.workloads import build_problem, rank1_space
 from oracle.pyoracle import BstOracle, Oracle
 
 pytestmark = pytest.mark.gpu
@@ -88,6 +88,30 @@ def test_shared_and_unshared_panels(eng, clusters, M, rank, R):
             got.append(plan.sigma(st.coeffs, prec))
         assert all(np.array_equal(g, got[0]) for g in got), prec
     eng.drop_plans()
+
+
+@pytest.mark.parametrize("R", [1, 2, 5, 9, 16])
+def test_row_sums_do_not_depend_on_the_number_of_rows(eng, R):
+    """One-row boxes below and above the count (2,048) from which a wavefront
+    takes a row alone: a row's sigma has the same bits in a bra space of 2,449
+    rows and in one of a few Fock blocks of it."""
+    p = build_problem(12, 3, 13, 24, seed=3, max_transfer=2)
+    ket = rank1_space(p, R=R, frac=1.0, seed=2)
+    assert len(ket) >= 2048
+    c = np.random.Generator(np.random.PCG64(R)).normal(size=(len(ket), R))
+    ham, ops = eng.ham(p.clustered_ham), eng.ops(p.cluster_ops)
+    dket = _lib.DeviceSpace.tpsci(eng.ctx, ket)
+    whole = _lib.Plan.create_pair(eng.ctx, ham, ops, _lib.DeviceSpace.tpsci(eng.ctx, ket), dket).sigma(c)
+    few = TPSCIstate(ket.N, R)
+    few.fock, few.fock_start = ket.fock[:9], ket.fock_start[:10]
+    few.cfg = ket.cfg[:few.fock_start[-1]]
+    few.coeffs = np.zeros((len(few.cfg), R))
+    part = _lib.Plan.create_pair(eng.ctx, ham, ops, _lib.DeviceSpace.tpsci(eng.ctx, few), dket).sigma(c)
+    print(len(ket), len(few), flush=True)
+    assert np.array_equal(part, whole[:len(few)])
+    ref = Oracle(flatten_ops(p.cluster_ops, cluster_sizes_of(p.cluster_ops)),
+                 flatten_ham(p.clustered_ham), ket).sigma(c)
+    assert np.abs(whole - ref).max() < 1e-12 * np.abs(ref).max()
 
 
 @pytest.mark.parametrize("shift", [0, 1, 5])
