@@ -756,7 +756,8 @@ int fcg_plan_set_apply_variant(fcg_plan_t pl, int precision, int R, int multi, i
 // root count (at most the tuned maximum), each variant of each apply kernel
 // runs twice on the caller's operands and the faster second run wins.  The
 // variants compute identical results, so the outputs of the timing runs are
-// simply overwritten.
+// simply overwritten -- unless they overlap c, which every run reads: such a
+// call takes the default variants and leaves the timing to a later one.
 static int tune_apply(fcg_ctx *ctx, fcg_plan *pl, int R, const double *c, double *s,
                       int precision, void *ci) {
   int nm = 1, nr = 1, max_r = 0;
@@ -793,6 +794,21 @@ static int tune_apply(fcg_ctx *ctx, fcg_plan *pl, int R, const double *c, double
   return FCG_OK;
 }
 
+// the variants of this call: the plan's, timed first where they are not yet
+static int apply_variants(fcg_ctx *ctx, fcg_plan *pl, int R, const double *c, double *s,
+                          int precision, void *ci, int *vm, int *vr) {
+  std::lock_guard<std::mutex> g(pl->tune_mu);
+  *vm = fcg_apply_default_variant(precision);
+  *vr = 0;
+  const bool apart = c + (int64_t)R * pl->ksp->nvar <= s || s + (int64_t)R * pl->sp->nvar <= c;
+  if (!pl->tuned[precision][R] && apart) TRY(tune_apply(ctx, pl, R, c, s, precision, ci));
+  if (pl->tuned[precision][R]) {
+    *vm = pl->tuned_vm[precision][R];
+    *vr = pl->tuned_vr[precision][R];
+  }
+  return FCG_OK;
+}
+
 extern "C" {
 
 int fcg_sigma_device(fcg_ctx_t ctx, fcg_plan_t pl, int R, const double *c_dev, double *s_dev,
@@ -823,13 +839,10 @@ int fcg_sigma_device(fcg_ctx_t ctx, fcg_plan_t pl, int R, const double *c_dev, d
     ctx->d_ci = p;
     ctx->ci_bytes = n * 8;
   }
-  {
-    std::lock_guard<std::mutex> g(pl->tune_mu);
-    if (!pl->tuned[precision][R])
-      TRY(tune_apply(ctx, pl, R, c_dev, s_dev, precision, ctx->d_ci));
-  }
-  FCG_HIP(fcg_launch_apply(pl, R, c_dev, s_dev, precision, ctx->stream, ctx->ev0,
-                           pl->tuned_vm[precision][R], pl->tuned_vr[precision][R], ctx->d_ci),
+  int vm, vr;
+  TRY(apply_variants(ctx, pl, R, c_dev, s_dev, precision, ctx->d_ci, &vm, &vr));
+  FCG_HIP(fcg_launch_apply(pl, R, c_dev, s_dev, precision, ctx->stream, ctx->ev0, vm, vr,
+                           ctx->d_ci),
           ctx);
   FCG_HIP(hipEventRecord(ctx->ev1, ctx->stream), ctx);
   ctx->last_launches = 2;
@@ -865,13 +878,9 @@ int fcg_sigma_device_noalloc(fcg_ctx_t ctx, fcg_plan_t pl, int R, const double *
   }
   (void)hipSetDevice(ctx->device);
   fcg_plan_note_user(pl, ctx);  // capacity reserved at plan creation
-  {
-    std::lock_guard<std::mutex> g(pl->tune_mu);
-    if (!pl->tuned[precision][R])
-      TRY(tune_apply(ctx, pl, R, c_dev, s_dev, precision, ctx->noalloc_scratch));
-  }
-  FCG_HIP(fcg_launch_apply(pl, R, c_dev, s_dev, precision, ctx->stream, ctx->ev0,
-                           pl->tuned_vm[precision][R], pl->tuned_vr[precision][R],
+  int vm, vr;
+  TRY(apply_variants(ctx, pl, R, c_dev, s_dev, precision, ctx->noalloc_scratch, &vm, &vr));
+  FCG_HIP(fcg_launch_apply(pl, R, c_dev, s_dev, precision, ctx->stream, ctx->ev0, vm, vr,
                            ctx->noalloc_scratch),
           ctx);
   FCG_HIP(hipEventRecord(ctx->ev1, ctx->stream), ctx);

@@ -131,3 +131,24 @@ def test_sigma_over_its_vector(eng, shift):
     eng.ctx.synchronize()
     assert np.array_equal(buf[:n].cpu().numpy(), ref)
     eng.drop_plans()
+
+
+@pytest.mark.parametrize("prec,R", [("fp64", 1), ("fp64", 3), ("fp32", 2)])
+def test_first_sigma_over_its_vector(eng, prec, R):
+    """The same on a plan's first sigma, whose timing runs must not read what
+    they have written."""
+    p = build_problem(12, 3, 4, 24, seed=4, max_transfer=1)
+    st = TPSCIstate.full_blocks(p.bases, p.focks, R=R)
+    c = np.random.Generator(np.random.PCG64(1)).normal(size=(len(st), R))
+    ref = eng.tpsci_plan(st, p.cluster_ops, p.clustered_ham, precisions=("fp64", prec)).sigma(c, prec)
+    eng.drop_plans()
+    plan = eng.tpsci_plan(st, p.cluster_ops, p.clustered_ham, precisions=("fp64", prec))
+    buf = torch.from_numpy(np.ascontiguousarray(c.T)).to("cuda:0")
+    torch.cuda.synchronize()
+    plan.sigma_device(buf.data_ptr(), buf.data_ptr(), R, prec)
+    eng.ctx.synchronize()
+    assert np.array_equal(buf.cpu().numpy().T, ref)
+    assert plan.apply_variant(prec, R) == (-1, -1)  # not timed yet
+    assert np.array_equal(plan.sigma(c, prec), ref)
+    assert min(plan.apply_variant(prec, R)) >= 0
+    eng.drop_plans()
