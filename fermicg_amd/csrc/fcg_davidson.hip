@@ -30,8 +30,7 @@
 
 namespace {
 
-constexpr int GT = 8;             // Gram output tile (GT x GT per workgroup)
-constexpr int GROWS = 128;        // rows staged in LDS per step
+constexpr int GL = 8;             // Gram output tile: GL x GL lanes, NB x NB outputs each
 constexpr int GTHR = 256;         // threads of a Gram workgroup
 constexpr int64_t GCHUNK = 4096;  // rows per split-K chunk
 constexpr int EMAX = 96;          // largest subspace whose eigenproblem runs on the GPU
@@ -68,14 +67,22 @@ __global__ void k_precond(int64_t n, int R, const double *hd, const double *thet
 // stages meanwhile.  At n = 9,125 (24 x 2 outputs) 224 us -> 28 us; one workgroup
 // per chunk with every output, 16 of them per thread, staged 64 columns
 // whether they existed or not and waited on LDS for each row.
+// With many workgroups (large n, large subspaces) the chains' LDS reads and
+// the tiles' reloads of V and W bound it instead: NB = 2 then gives a lane
+// 2 x 2 outputs, half the reads of each per multiply-add.  n = 2,000,089, us:
+// 96 x 96 outputs 3,017 (8 x 8 tiles 5,127; 16 x 16 tiles of one output per
+// thread 4,881), 64 x 16 368 (586; 952 with one workgroup per chunk).
 constexpr int GAHEAD = 4;  // stages loaded ahead
 static_assert(GAHEAD % 2 == 0, "stage d uses LDS buffer d & 1 in every round");
-constexpr int GB = 8;      // row pairs read from LDS at a time
 constexpr int GPAD = 2;  // doubles between staged columns: 16-byte aligned, banks spread
+template <int NB>
 __global__ __launch_bounds__(GTHR, 1) void k_gram_partial(int64_t n,
                                                        const double *__restrict__ V,
                                                        int mv, const double *__restrict__ W,
                                                        int mw, double *__restrict__ part) {
+  constexpr int GT = GL * NB;
+  constexpr int GROWS = 128 / NB;  // rows staged in LDS per step
+  constexpr int GB = 8 / NB;       // row pairs read from LDS at a time
   __shared__ __align__(16) double sX[2][2 * GT][GROWS + GPAD];
   const int tid = threadIdx.x;
   const int i0 = blockIdx.y * GT, j0 = blockIdx.z * GT;
@@ -113,24 +120,29 @@ __global__ __launch_bounds__(GTHR, 1) void k_gram_partial(int64_t n,
   store(r_begin, v[0], 0);
   load(r_begin + GAHEAD * GROWS, v[0]);
   __syncthreads();
-  const int i = tid % GT, j = (tid / GT) % GT;
-  double acc = 0.0;
+  // outputs (i + GL a, j + GL b)
+  const int i = tid % GL, j = (tid / GL) % GL;
+  double acc[NB][NB];
+#pragma unroll
+  for (int a = 0; a < NB; a++)
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[a][b] = 0.0;
   for (int64_t r0 = r_begin; r0 < r_end; r0 += GAHEAD * GROWS) {
 #pragma unroll
     for (int d = 0; d < GAHEAD; d++) {
       const int buf = d & 1;
-      if (tid < GT * GT) {
-        const double2 *a = reinterpret_cast<const double2 *>(sX[buf][i]);
-        const double2 *b = reinterpret_cast<const double2 *>(sX[buf][GT + j]);
-        // eight row pairs read ahead of the eight in use: left to itself the
+      if (tid < GL * GL) {
+        // GB row pairs read ahead of the GB in use: left to itself the
         // compiler reads each pair where it is used and waits for LDS
-        double2 x[2][GB], y[2][GB];
-        auto fetch = [&](int p, double2 (&u)[GB], double2 (&w)[GB]) {
+        double2 x[2][GB][NB], y[2][GB][NB];
+        auto fetch = [&](int p, double2 (&u)[GB][NB], double2 (&w)[GB][NB]) {
 #pragma unroll
-          for (int k = 0; k < GB; k++) {
-            u[k] = a[p + k];
-            w[k] = b[p + k];
-          }
+          for (int k = 0; k < GB; k++)
+#pragma unroll
+            for (int a = 0; a < NB; a++) {
+              u[k][a] = reinterpret_cast<const double2 *>(sX[buf][i + GL * a])[p + k];
+              w[k][a] = reinterpret_cast<const double2 *>(sX[buf][GT + j + GL * a])[p + k];
+            }
         };
         fetch(0, x[0], y[0]);
 #pragma unroll
@@ -140,8 +152,14 @@ __global__ __launch_bounds__(GTHR, 1) void k_gram_partial(int64_t n,
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int k = 0; k < GB; k++) {
-            acc += x[h][k].x * y[h][k].x;
-            acc += x[h][k].y * y[h][k].y;
+#pragma unroll
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+              for (int b = 0; b < NB; b++) acc[a][b] += x[h][k][a].x * y[h][k][b].x;
+#pragma unroll
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+              for (int b = 0; b < NB; b++) acc[a][b] += x[h][k][a].y * y[h][k][b].y;
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -153,8 +171,15 @@ __global__ __launch_bounds__(GTHR, 1) void k_gram_partial(int64_t n,
       __syncthreads();
     }
   }
-  if (tid < GT * GT && i < nv && j < nw)
-    part[(int64_t)blockIdx.x * mv * mw + (i0 + i) + (int64_t)mv * (j0 + j)] = acc;
+  if (tid < GL * GL) {
+#pragma unroll
+    for (int a = 0; a < NB; a++)
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+        if (i + GL * a < nv && j + GL * b < nw)
+          part[(int64_t)blockIdx.x * mv * mw + (i0 + i + GL * a) +
+               (int64_t)mv * (j0 + j + GL * b)] = acc[a][b];
+  }
 }
 
 // out[i + ld*j] = sum over chunks of part[chunk][i + ma*j], one wavefront per
@@ -434,9 +459,22 @@ int gram(Dav &d, const double *A, int ma, const double *B, int mb, double *dev_o
          std::vector<double> *host_out, int ld = 0) {
   fcg_ctx *ctx = d.ctx;
   if (ld <= 0) ld = ma;
-  const dim3 grid((unsigned)d.nchunk, (unsigned)((ma + GT - 1) / GT),
-                  (unsigned)((mb + GT - 1) / GT));
-  hipLaunchKernelGGL(k_gram_partial, grid, dim3(GTHR), 0, ctx->stream, d.n, A, ma, B, mb, d.part);
+  auto partial = [&](auto nb) {
+    constexpr int NB = decltype(nb)::value, GT = GL * NB;
+    const dim3 grid((unsigned)d.nchunk, (unsigned)((ma + GT - 1) / GT),
+                    (unsigned)((mb + GT - 1) / GT));
+    hipLaunchKernelGGL(k_gram_partial<NB>, grid, dim3(GTHR), 0, ctx->stream, d.n, A, ma, B, mb,
+                       d.part);
+  };
+  // 2 x 2 outputs per lane take 68 us a round of workgroups (two per CU)
+  // against 30, so they pay from about two rounds of 8 x 8 tiles on, and
+  // where they are at least three times fewer (no side of one tile): us at
+  // 1,040 / 260 workgroups 99 / 84, 576 / 144 64 / 71, 978 / 489 84 / 87
+  auto groups = [&](int t) { return (int64_t)d.nchunk * ((ma + t - 1) / t) * ((mb + t - 1) / t); };
+  if (groups(GL) >= 960 && groups(GL) >= 3 * groups(2 * GL))
+    partial(std::integral_constant<int, 2>{});
+  else
+    partial(std::integral_constant<int, 1>{});
   const int cnt = ma * mb;
   hipLaunchKernelGGL(k_gram_reduce, dim3((unsigned)cnt), dim3(64), 0, ctx->stream, d.nchunk, ma,
                      cnt, d.part, dev_out, ld);

@@ -1,8 +1,9 @@
 """Davidson where its tall-skinny products have edges: spaces around a stage
-of rows (128) and a round of four stages, and root counts below and above an
-output tile (8 columns).
+of rows (128) and a round of four stages, root counts below and above an
+output tile (8 columns), spaces of several row chunks (4,096) and products
+large enough for 2 x 2 outputs per lane.
 
-Reference: the eigenvalues and residuals of the dense H of the same space
+Reference up to one chunk: the eigenvalues and residuals of the dense H of the same space
 (build_full_H, symmetrised).  Bars: the solver stops at a residual norm of
 1e-9, so each energy lies within 1e-9 of an eigenvalue of H, and the residual
 recomputed here within 2e-9 (its own rounding is 1e-13); orthonormal vectors to
@@ -13,7 +14,7 @@ import pytest
 
 from fermicg_amd.state import TPSCIstate
 from fermicg_amd.tpsci import Engine, build_full_H
-from fermicg_amd.workloads import tpsci_small
+from fermicg_amd.workloads import build_problem, tpsci_small
 
 pytestmark = pytest.mark.gpu
 
@@ -52,4 +53,25 @@ def test_davidson_sizes(problem, n, R, ss):
     w = np.linalg.eigvalsh(H)
     assert max(np.abs(w - x).min() for x in e) < 1e-9
     assert np.linalg.norm(H @ v - v * e, axis=0).max() < 2e-9
+    assert np.abs(v.T @ v - np.eye(R)).max() < 1e-11
+
+
+@pytest.mark.parametrize("M,R,ss", [(4, 2, 24), (4, 16, 12), (5, 3, 10), (5, 16, 16)])
+def test_davidson_several_chunks(M, R, ss):
+    """4,672 and 9,125 rows.  16 roots reach subspaces of 192 and 256 columns,
+    whose m x m products take 2 x 2 outputs per lane.  A residual norm (with
+    the plan's own sigma) below 2e-9 puts an eigenvalue within 2e-9."""
+    p = build_problem(12, 3, M, 24, seed=3, max_transfer=2)
+    st = TPSCIstate.full_blocks(p.bases, p.focks, R=R)
+    eng = Engine(0)
+    pl = eng.tpsci_plan(st, p.cluster_ops, p.clustered_ham)
+    n = len(st)
+    v0 = np.zeros((n, R))
+    v0[np.argsort(pl.diagonal())[:R], np.arange(R)] = 1.0
+    v0 += 0.001 * np.random.Generator(np.random.PCG64(n)).normal(size=(n, R))
+    e, v, stats = pl.davidson(v0, conv_thresh=1e-9, max_iter=500, max_ss_vecs=ss)
+    print("n", n, "R", R, stats["iterations"], stats["converged"], flush=True)
+    assert stats["converged"]
+    assert np.abs(np.sort(e) - e).max() < 1e-9
+    assert np.linalg.norm(pl.sigma(v) - v * e, axis=0).max() < 2e-9
     assert np.abs(v.T @ v - np.eye(R)).max() < 1e-11
