@@ -754,18 +754,21 @@ int fcg_plan_set_apply_variant(fcg_plan_t pl, int precision, int R, int multi, i
 
 // Autotuning of the apply: on the first sigma of a plan for a precision and
 // root count (at most the tuned maximum), each variant of each apply kernel
-// runs twice on the caller's operands and the faster second run wins.  The
-// variants compute identical results, so the outputs of the timing runs are
-// simply overwritten -- unless they overlap c, which every run reads: such a
-// call takes the default variants and leaves the timing to a later one.
+// runs twice on the caller's operands and the faster second run wins; one
+// whose first run is a fifth slower than the best so far (and by more than
+// a cold start, 50 us) is not run twice.  The variants compute identical
+// results, so the outputs of the timing runs are simply overwritten -- unless
+// they overlap c, which every run reads: such a call takes the default
+// variants and leaves the timing to a later one.
 static int tune_apply(fcg_ctx *ctx, fcg_plan *pl, int R, const double *c, double *s,
                       int precision, void *ci) {
   int nm = 1, nr = 1, max_r = 0;
   fcg_apply_n_variants(&nm, &nr, &max_r);
   int best_m = fcg_apply_default_variant(precision), best_r = 0;
   if (R <= max_r) {
-    auto time_it = [&](int vm, int vr, int parts, float *ms) -> int {
+    auto time_it = [&](int vm, int vr, int parts, float best, float *ms) -> int {
       for (int rep = 0; rep < 2; rep++) {
+        if (rep == 1 && *ms > 1.2f * best && *ms > best + 0.05f) break;
         FCG_HIP(fcg_launch_apply(pl, R, c, s, precision, ctx->stream, ctx->ev0, vm, vr, ci,
                                  parts),
                 ctx);
@@ -777,14 +780,15 @@ static int tune_apply(fcg_ctx *ctx, fcg_plan *pl, int R, const double *c, double
     };
     float best = 1e30f, t = 0.f;
     if (pl->n_multi > 0)
-      for (int vm = 0; vm < nm; vm++) {
-        TRY(time_it(vm, 0, 1, &t));
+      for (int k = 0; k < nm; k++) {  // the default first
+        const int vm = (fcg_apply_default_variant(precision) + k) % nm;
+        TRY(time_it(vm, 0, 1, best, &t));
         if (t < best) { best = t; best_m = vm; }
       }
     best = 1e30f;
     if (pl->n_single_slots > 0)
       for (int vr = 0; vr < nr; vr++) {
-        TRY(time_it(best_m, vr, 2, &t));
+        TRY(time_it(best_m, vr, 2, best, &t));
         if (t < best) { best = t; best_r = vr; }
       }
   }
