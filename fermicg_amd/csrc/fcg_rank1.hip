@@ -156,11 +156,13 @@ struct R1Ready {
 // and a pair's terms prepared TS at a time by one thread per (term, cluster);
 // W_a and e come from W_ab instead of from V again; the cross part W_ab u_b is
 // formed once per (a, p) instead of once per state of a; and the state
-// blocks' w_ij = W_a . Γ_a[:, i, j] are spread over all threads.  Four
-// barriers per term.  102,673 configurations of 6 clusters, 2 roots, FP64:
+// blocks' w_ij = W_a . Γ_a[:, i, j] are spread over all threads.  Barriers per
+// term: three up to W_a and z_a, one after each cluster's tile of w_ij and one
+// before every tile but the first: 4, 6, 8, 10 for one to four clusters whose
+// w_ij fit one tile each.  102,673 configurations of 6 clusters, 2 roots, FP64:
 // 508 ms with each bra state forming its own cross part and every W_a summing V,
 // 65 ms without, 50 ms with the shape in scalar registers and eight loads in
-// flight per dot product.
+// flight per dot product; 2,000,089 of 8 clusters, 4 roots: 7.6 s.
 template <typename T, bool DIAG>
 __global__ __launch_bounds__(RT) void k_rank1(R1Args<T> a) {
   __shared__ T sY[LMAX * RC];
