@@ -756,7 +756,7 @@ int fcg_plan_set_apply_variant(fcg_plan_t pl, int precision, int R, int multi, i
 // root count (at most the tuned maximum), each variant of each apply kernel
 // runs twice on the caller's operands and the faster second run wins; one
 // whose first run is a fifth slower than the best so far (and by more than
-// a cold start, 50 us) is not run twice.  The variants compute identical
+// a cold start, 30 us) is not run twice.  The variants compute identical
 // results, so the outputs of the timing runs are simply overwritten -- unless
 // they overlap c, which every run reads: such a call takes the default
 // variants and leaves the timing to a later one.
@@ -768,7 +768,7 @@ static int tune_apply(fcg_ctx *ctx, fcg_plan *pl, int R, const double *c, double
   if (R <= max_r) {
     auto time_it = [&](int vm, int vr, int parts, float best, float *ms) -> int {
       for (int rep = 0; rep < 2; rep++) {
-        if (rep == 1 && *ms > 1.2f * best && *ms > best + 0.05f) break;
+        if (rep == 1 && *ms > 1.2f * best && *ms > best + 0.03f) break;
         FCG_HIP(fcg_launch_apply(pl, R, c, s, precision, ctx->stream, ctx->ev0, vm, vr, ci,
                                  parts),
                 ctx);
